@@ -138,8 +138,11 @@ typedef struct ion_kernel_constants {
 /* Field-update arithmetic (build-side option, no reference counterpart):
  *   ION_FIELD_EXACT: the reference's r/|r|^3 with correctly rounded sqrt and
  *                    division and unfused accumulation (default);
- *   ION_FIELD_FAST:  hardware reciprocal square root and fused accumulation,
- *                    within a stated relative tolerance of EXACT. */
+ *   ION_FIELD_FAST:  hardware reciprocal square root and fused accumulation;
+ *                    with many sources, those far from a block of cells are
+ *                    summed at sample points of the block and interpolated
+ *                    (error below the rounding of the sums); within a
+ *                    relative tolerance of 1e-5 of EXACT (2-norm). */
 typedef enum { ION_FIELD_EXACT = 0, ION_FIELD_FAST = 1 } ion_field_mode;
 
 /* Accumulated GPU time per kernel (hipEvent pairs on the handle's stream),
@@ -245,8 +248,9 @@ typedef struct ion_field_buffers {
  * (update_e_b_dynamic, src/kernels/sim_kernels.cl:897-993) on caller-owned
  * device buffers; E_dyn and B_dyn are bit-identical to ion_compute_fields on
  * the same inputs. It allocates nothing: the compacted LOD source list lives
- * in a static device array of ION_NOALLOC_MAX_SOURCES entries (1 MiB), one
- * per GPU, held until the process ends. cfg supplies the lattice, the LOD
+ * in a static device array of ION_NOALLOC_MAX_SOURCES entries (1 MiB), with
+ * the field samples of ION_FIELD_FAST beside it (64 MiB), one per GPU, held
+ * until the process ends. cfg supplies the lattice, the LOD
  * depth (<= 5) and the units (KE, KMU); ext_magneto_hydro, FP32/FP16S/FP16C
  * (fields are float). field_mode: ION_FIELD_EXACT or ION_FIELD_FAST.
  * Enqueued on `stream` (a hipStream_t; NULL: the null stream) without

@@ -1,5 +1,7 @@
 // gfx950 kernels of the dynamic E/B field update (update_e_b_dynamic,
-// sim_kernels.cl:897-993) and of the float64 conservation sums.
+// sim_kernels.cl:897-993) and of the float64 conservation sums: the source
+// list, the sum over it in EXACT and FP64 arithmetic and wherever there is a
+// near field (field_fast.hip has the rest of FAST), the judge's reductions.
 //
 // The field at every fluid cell is a sum over the level-of-detail (LOD)
 // sources of the own domain: E += q r/|r|^3, B += q v x r/|r|^3. The
@@ -10,6 +12,8 @@
 #include <hip/hip_runtime.h>
 
 #include "cr_math.hpp"
+#include "field_fast.hpp"
+#include "judge.hpp"
 #include "kernels.hpp"
 
 namespace ion {
@@ -17,7 +21,9 @@ namespace ion {
 // ---------------------------------------------------------------------------
 // Source list: LOD indices d in [lo, hi) with a non-zero charge, in index
 // order. A source of zero charge adds exactly zero to every cell, so
-// dropping it leaves all fields unchanged.
+// dropping it leaves all fields unchanged. *mode (if not null): whether the
+// multilevel field update may be used, i.e. there are enough sources and none
+// is infinite, NaN or so large that a partial sum could overflow.
 // ---------------------------------------------------------------------------
 // 4-vectors of the arithmetic type; the 4th component of a source's vd
 // carries its LOD index (float: the bits, double: the value, exact below 2^53).
@@ -46,10 +52,11 @@ __global__ void __launch_bounds__(1024) k_prep_sources(const typename V4F<R>::T*
                                                        uint32_t hi, uint32_t nd, R dsx, R dsy, R dsz,
                                                        typename V4F<R>::T* __restrict__ src_pq,
                                                        typename V4F<R>::T* __restrict__ src_vd,
-                                                       uint32_t* __restrict__ count) {
+                                                       uint32_t* __restrict__ count, uint32_t* __restrict__ mode) {
     __shared__ uint32_t wave_tot[16];
     __shared__ uint32_t base_sh;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
+    bool wild = false;
     if (tid == 0) base_sh = 0;
     __syncthreads();
     for (uint32_t c0 = lo; c0 < hi; c0 += 1024) {
@@ -67,6 +74,7 @@ __global__ void __launch_bounds__(1024) k_prep_sources(const typename V4F<R>::T*
         uint32_t off = base_sh;
         for (uint32_t k = 0; k < wv; k++) off += wave_tot[k];
         if (keep) {
+            wild |= !(fabs(e.x) * (R(1) + fabs(e.y) + fabs(e.z) + fabs(e.w)) < R(1e30f));
             const uint32_t o = off + pre;
             const uint32_t t = d % (nd * nd);
             // lod_coordinates, sim_kernels.cl:442-447
@@ -84,7 +92,11 @@ __global__ void __launch_bounds__(1024) k_prep_sources(const typename V4F<R>::T*
         }
         __syncthreads();
     }
-    if (tid == 0) *count = base_sh;
+    const bool any_wild = __syncthreads_or(wild);
+    if (tid == 0) {
+        *count = base_sh;
+        if (mode != nullptr) *mode = base_sh >= ML_MIN_SOURCES && !any_wild;
+    }
 }
 
 constexpr uint32_t FIELD_TILE = 512;
@@ -105,29 +117,6 @@ __device__ __forceinline__ void interact_exact(R q, R vx, R vy, R vz, R rx, R ry
     bx = bx + q * crx;
     by = by + q * cry;
     bz = bz + q * crz;
-}
-
-// Judge partials of a block: the work-items' four sums (E error, E norm,
-// B error, B norm) reduced in a fixed order (wavefront tree, then the
-// wavefronts in order) into partial[blockIdx.x][4], in double.
-__device__ __forceinline__ void judge_block_sums(const float v[4], double* partial) {
-    __shared__ double jsh[16][4];
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    double d[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        d[k] = (double)v[k];
-        for (int o = 32; o >= 1; o >>= 1) d[k] += __shfl_down(d[k], o, 64);
-    }
-    if (lane == 0)
-#pragma unroll
-        for (int k = 0; k < 4; k++) jsh[wv][k] = d[k];
-    __syncthreads();
-    if (threadIdx.x < 4) {
-        double t = 0.0;
-        for (uint32_t w = 0; w < (blockDim.x + 63u) / 64u; w++) t += jsh[w][threadIdx.x];
-        partial[(size_t)blockIdx.x * 4 + threadIdx.x] = t;
-    }
 }
 
 template <bool FAST, bool NEAR, int CPT>
@@ -318,7 +307,7 @@ __global__ void __launch_bounds__(FIELD_BLOCK) k_update_e_b_f64(FieldArgs a) {
     bd[2 * N + n] = bs[2 * N + n] + kmu * bz;
 }
 
-// The field update on LOD-aligned tiles, FAST or EXACT arithmetic. A block covers
+// The field update on LOD-aligned tiles, EXACT arithmetic. A block covers
 // (ROW*TX) x TY x TZ cells inside one top-level LOD block, so the own-LOD
 // skip is the same for every cell of the block: a wave-uniform branch on the
 // source's LOD index. Each thread owns ROW consecutive cells of one row: the
@@ -336,7 +325,7 @@ __global__ void __launch_bounds__(FIELD_BLOCK) k_update_e_b_f64(FieldArgs a) {
 // Held to 80 VGPRs (6 wavefronts per SIMD, no spills; the sweep's VALU
 // instructions are the same as at 105 VGPRs) so that the scalar loads at the
 // top of each source's iteration hide behind the other wavefronts.
-template <int ROW, bool FAST>
+template <int ROW>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
     __shared__ float s_epi[ROW * 256];
@@ -379,8 +368,7 @@ k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
         // arithmetic, so their latency hides behind it
         float4 vd_next = svd[s0], pq_next = spq[s0];
         // one source per iteration: the compiler then lays the ROW cells'
-        // chains side by side (measured at 256^3, FAST: 17.0 ms against
-        // 18.1 ms with two sources per iteration and 17.5 ms with four)
+        // chains side by side
 #pragma unroll 1
         for (uint32_t s = s0; s < s1; s++) {
             const float4 vd = vd_next, pq = pq_next;
@@ -388,42 +376,24 @@ k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
             vd_next = svd[sn];
             pq_next = spq[sn];
             const float ry = py - pq.y, rz = pz - pq.z;
-            if constexpr (FAST) {
-                const float syz = __builtin_fmaf(ry, ry, rz * rz);
-                const float cx = __builtin_fmaf(vd.y, rz, -(vd.z * ry));  // (v x r).x
-                const float m1 = vd.x * rz, m2 = vd.x * ry;
+            // interact_exact with r_y^2, r_z^2 hoisted: pre = r / |r|^3,
+            // e += q pre, b += q (v x pre), every operation rounded on its own
+            const float ry2 = ry * ry, rz2 = rz * rz;
+            const float q = pq.w;
 #pragma unroll
-                for (int k = 0; k < ROW; k++) {
-                    const float rx = px[k] - pq.x;
-                    const float inv = __builtin_amdgcn_rsqf(__builtin_fmaf(rx, rx, syz));
-                    const float t = pq.w * (inv * inv * inv);
-                    ex[k] = __builtin_fmaf(t, rx, ex[k]);
-                    ey[k] = __builtin_fmaf(t, ry, ey[k]);
-                    ez[k] = __builtin_fmaf(t, rz, ez[k]);
-                    bxa[k] = __builtin_fmaf(t, cx, bxa[k]);
-                    bya[k] = __builtin_fmaf(t, __builtin_fmaf(vd.z, rx, -m1), bya[k]);  // (v x r).y
-                    bza[k] = __builtin_fmaf(t, __builtin_fmaf(-vd.y, rx, m2), bza[k]);  // (v x r).z
-                }
-            } else {
-                // interact_exact with r_y^2, r_z^2 hoisted: pre = r / |r|^3,
-                // e += q pre, b += q (v x pre), every operation rounded on its own
-                const float ry2 = ry * ry, rz2 = rz * rz;
-                const float q = pq.w;
-#pragma unroll
-                for (int k = 0; k < ROW; k++) {
-                    const float rx = px[k] - pq.x;
-                    const float sm = sqrt_cr((rx * rx + ry2) + rz2);
-                    const float cbm = (sm * sm) * sm;
-                    const float prx = div_cr(rx, cbm), pry = div_cr(ry, cbm), prz = div_cr(rz, cbm);
-                    ex[k] = ex[k] + q * prx;
-                    ey[k] = ey[k] + q * pry;
-                    ez[k] = ez[k] + q * prz;
-                    const float crx = vd.y * prz - vd.z * pry, cry = vd.z * prx - vd.x * prz,
-                                crz = vd.x * pry - vd.y * prx;
-                    bxa[k] = bxa[k] + q * crx;
-                    bya[k] = bya[k] + q * cry;
-                    bza[k] = bza[k] + q * crz;
-                }
+            for (int k = 0; k < ROW; k++) {
+                const float rx = px[k] - pq.x;
+                const float sm = sqrt_cr((rx * rx + ry2) + rz2);
+                const float cbm = (sm * sm) * sm;
+                const float prx = div_cr(rx, cbm), pry = div_cr(ry, cbm), prz = div_cr(rz, cbm);
+                ex[k] = ex[k] + q * prx;
+                ey[k] = ey[k] + q * pry;
+                ez[k] = ez[k] + q * prz;
+                const float crx = vd.y * prz - vd.z * pry, cry = vd.z * prx - vd.x * prz,
+                            crz = vd.x * pry - vd.y * prx;
+                bxa[k] = bxa[k] + q * crx;
+                bya[k] = bya[k] + q * cry;
+                bza[k] = bza[k] + q * crz;
             }
         }
     };
@@ -543,15 +513,16 @@ __global__ void __launch_bounds__(256) k_sum_f64(const T* __restrict__ x, const 
 }
 
 hipError_t launch_prep_sources(const void* qu_lod, bool f64, uint32_t lo, uint32_t hi, uint32_t nx, uint32_t ny,
-                               uint32_t nz, uint32_t D, void* src_pq, void* src_vd, uint32_t* count, hipStream_t s) {
+                               uint32_t nz, uint32_t D, void* src_pq, void* src_vd, uint32_t* count, uint32_t* mode,
+                               hipStream_t s) {
     const uint32_t nd = 1u << D;
     const float dx = (float)(nx / nd), dy = (float)(ny / nd), dz = (float)(nz / nd);
     if (f64)
         hipLaunchKernelGGL(k_prep_sources<double>, dim3(1), dim3(1024), 0, s, (const double4*)qu_lod, lo, hi, nd,
-                           (double)dx, (double)dy, (double)dz, (double4*)src_pq, (double4*)src_vd, count);
+                           (double)dx, (double)dy, (double)dz, (double4*)src_pq, (double4*)src_vd, count, mode);
     else
         hipLaunchKernelGGL(k_prep_sources<float>, dim3(1), dim3(1024), 0, s, (const float4*)qu_lod, lo, hi, nd, dx,
-                           dy, dz, (float4*)src_pq, (float4*)src_vd, count);
+                           dy, dz, (float4*)src_pq, (float4*)src_vd, count, mode);
     return hipGetLastError();
 }
 
@@ -578,10 +549,18 @@ static FieldShape field_shape(const FieldArgs& a, bool fast) {
     return FieldShape{0, 0, 0, 0, (uint32_t)((a.N + per - 1) / per)};
 }
 
-uint32_t field_blocks(const FieldArgs& a, bool fast) { return field_shape(a, fast).blocks; }
+uint32_t field_blocks(const FieldArgs& a, bool fast) {
+    MlArgs m;
+    if (fast && ml_plan(a, &m)) return ml_blocks(m);
+    return field_shape(a, fast).blocks;
+}
 
 hipError_t launch_update_e_b(const FieldArgs& a, bool fast, hipStream_t s) {
     constexpr int CPT_EXACT = 1, CPT_FAST = 2;
+    if (fast && !a.f64 && !a.near) {
+        MlArgs m;
+        return ml_plan(a, &m) ? launch_field_fast(m, s) : hipErrorInvalidValue;
+    }
     const FieldShape sh = field_shape(a, fast);
     if (a.f64) {
         if (a.judge != nullptr) return hipErrorInvalidValue;
@@ -591,19 +570,13 @@ hipError_t launch_update_e_b(const FieldArgs& a, bool fast, hipStream_t s) {
     if (sh.row) {
         const uint32_t TX = sh.TX, TY = sh.TY, TZ = sh.TZ;
         const dim3 g(sh.blocks), bl(TX * TY * TZ);
-        if (fast) {
-            if (sh.row == 8) hipLaunchKernelGGL((k_update_e_b_tiled<8, true>), g, bl, 0, s, a, TX, TY, TZ);
-            else hipLaunchKernelGGL((k_update_e_b_tiled<4, true>), g, bl, 0, s, a, TX, TY, TZ);
-        } else {
-            if (sh.row == 8) hipLaunchKernelGGL((k_update_e_b_tiled<8, false>), g, bl, 0, s, a, TX, TY, TZ);
-            else hipLaunchKernelGGL((k_update_e_b_tiled<4, false>), g, bl, 0, s, a, TX, TY, TZ);
-        }
+        if (sh.row == 8) hipLaunchKernelGGL((k_update_e_b_tiled<8>), g, bl, 0, s, a, TX, TY, TZ);
+        else hipLaunchKernelGGL((k_update_e_b_tiled<4>), g, bl, 0, s, a, TX, TY, TZ);
         return hipGetLastError();
     }
     const dim3 g(sh.blocks), b(FIELD_BLOCK);
     if (fast) {
-        if (a.near) hipLaunchKernelGGL((k_update_e_b<true, true, CPT_FAST>), g, b, 0, s, a);
-        else hipLaunchKernelGGL((k_update_e_b<true, false, CPT_FAST>), g, b, 0, s, a);
+        hipLaunchKernelGGL((k_update_e_b<true, true, CPT_FAST>), g, b, 0, s, a);
     } else {
         if (a.near) hipLaunchKernelGGL((k_update_e_b<false, true, CPT_EXACT>), g, b, 0, s, a);
         else hipLaunchKernelGGL((k_update_e_b<false, false, CPT_EXACT>), g, b, 0, s, a);

@@ -16,6 +16,7 @@
 #include <string>
 #include <vector>
 
+#include "field_fast.hpp"
 #include "internal.hpp"
 #include "ionsolver.h"
 #include "kernels.hpp"
@@ -84,6 +85,7 @@ struct ion_handle {
     float4* src_pq = nullptr;
     float4* src_vd = nullptr;
     uint32_t* src_count = nullptr;
+    float* ml_ws = nullptr;  // workspace of the multilevel field update
     double* partials = nullptr;
     uint32_t n_partials = 1024;
     std::vector<void*> allocs;
@@ -252,7 +254,7 @@ int prep_sources(ion_handle* h) {
     const uint32_t hi = (uint32_t)h->n_lod, lo = (uint32_t)(h->n_lod - n_top);
     return timed(h, 2, [&] {
         return ion::launch_prep_sources(h->qu_lod, h->f64(), lo, hi, h->cfg.n_x, h->cfg.n_y, h->cfg.n_z, h->D,
-                                        h->src_pq, h->src_vd, h->src_count, h->stream);
+                                        h->src_pq, h->src_vd, h->src_count, (uint32_t*)h->ml_ws, h->stream);
     });
 }
 
@@ -285,6 +287,8 @@ ion::FieldArgs field_args(ion_handle* h) {
     f.kmu = h->kc.kmu;
     f.raw = h->field_raw;
     f.f64 = h->f64() ? 1u : 0u;
+    f.qu = (const float4*)h->qu_lod;
+    f.ml_ws = h->ml_ws;
     return f;
 }
 
@@ -597,6 +601,8 @@ int ion_create(const ion_config* cfg, ion_handle** out) {
         if ((rc = dalloc(h, (void**)&h->src_pq, n_top * 4 * rs))) return bail(rc);
         if ((rc = dalloc(h, (void**)&h->src_vd, n_top * 4 * rs))) return bail(rc);
         if ((rc = dalloc(h, (void**)&h->src_count, sizeof(uint32_t)))) return bail(rc);
+        ion::MlArgs ml;
+        if (ion::ml_plan(field_args(h), &ml) && (rc = dalloc(h, (void**)&h->ml_ws, ml.ws_floats * sizeof(float)))) return bail(rc);
         if (h->lod && (rc = dalloc(h, (void**)&h->lod_seg, (N / h->lod_bx) * 4 * rs))) return bail(rc);
         h->ecr = cfg->ext_subgrid_ecr != 0;
         if (h->ecr) {
@@ -869,10 +875,11 @@ int ion_compute_fields(ion_handle* h) {
 
 // Scratch of ion_update_e_b_noalloc: the compacted LOD sources (centre and
 // charge, then mean velocity and LOD index: ION_NOALLOC_MAX_SOURCES float4
-// each) followed by their count. Every GPU the library runs on holds its own
+// each) followed by their count, and the workspace of the multilevel field
+// update. Every GPU the library runs on holds its own
 // copy at its own address; host code uses that address (scratch_on_device),
 // never the array's name, which in host code is only a stand-in.
-static __device__ __align__(256) float4 scratch[2 * ION_NOALLOC_MAX_SOURCES + 16];
+static __device__ __align__(256) float4 scratch[2 * ION_NOALLOC_MAX_SOURCES + 16 + ion::ML_WS_FLOATS / 4];
 
 namespace {
 
@@ -935,9 +942,10 @@ int ion_update_e_b_noalloc(const ion_config* cfg, const ion_field_buffers* b, in
     float4* src_pq = s;
     float4* src_vd = s + ION_NOALLOC_MAX_SOURCES;
     uint32_t* count = (uint32_t*)(s + 2 * ION_NOALLOC_MAX_SOURCES);
+    float* ml_ws = (float*)(s + 2 * ION_NOALLOC_MAX_SOURCES + 16);
     hipStream_t st = (hipStream_t)stream;
     hipError_t e = ion::launch_prep_sources(b->qu_lod, false, lo, hi, cfg->n_x, cfg->n_y, cfg->n_z, D, src_pq, src_vd,
-                                            count, st);
+                                            count, (uint32_t*)ml_ws, st);
     if (e != hipSuccess) return fail(ION_ERR_DEVICE, std::string("source compaction: ") + hipGetErrorString(e));
     f.e_stat = b->e_stat;
     f.b_stat = b->b_stat;
@@ -958,6 +966,8 @@ int ion_update_e_b_noalloc(const ion_config* cfg, const ion_field_buffers* b, in
     f.kmu = k.kmu;
     f.raw = nullptr;
     f.f64 = 0u;
+    f.qu = (const float4*)b->qu_lod;
+    f.ml_ws = ml_ws;
     e = ion::launch_update_e_b(f, field_mode == ION_FIELD_FAST, st);
     if (e != hipSuccess) return fail(ION_ERR_DEVICE, std::string("field kernel: ") + hipGetErrorString(e));
     return ION_OK;
