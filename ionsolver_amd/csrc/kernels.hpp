@@ -73,11 +73,12 @@ struct FieldArgs {
     // the B components into judge[block][4] before writing its own fields
     double* judge;
     const float4* qu;       // LOD sums [n_lod]
-    float* ml_ws;           // workspace of the multilevel update (ml_workspace floats)
+    float* ml_ws;           // workspace of the multilevel update (MlArgs::ws_floats), or null
+    const uint32_t* mode;   // in it: whether the updates over all LOD blocks may be used [MODE_FAST, MODE_EXACT]
+    const float4* dense;    // in it: (q, v) at every LOD index
+    uint32_t second;        // set by launch_update_e_b: another kernel runs first
 };
-// Fewest charged sources for which the multilevel update is used (fast
-// arithmetic).
-constexpr uint32_t ML_MIN_SOURCES = 256;
+enum { MODE_FAST = 0, MODE_EXACT = 1 };
 // Number of blocks (judge partials) the field kernel launches for a.
 uint32_t field_blocks(const FieldArgs& a, bool fast);
 // Sums judge partials [nblocks][4] in a fixed order into out[4] (E err, E norm, B err, B norm).
@@ -99,7 +100,10 @@ hipError_t launch_codec(int store, int dir, const void* in, void* out, uint64_t 
 // kernels_field.hip
 hipError_t launch_prep_sources(const void* qu_lod, bool f64, uint32_t lo, uint32_t hi, uint32_t nx, uint32_t ny,
                                uint32_t nz, uint32_t D, void* src_pq, void* src_vd, uint32_t* count, uint32_t* mode,
-                               hipStream_t s);
+                               float4* dense, hipStream_t s);
+// Whether it may run an update over all LOD blocks (which reads mode and dense;
+// judge: with a.judge set).
+bool over_all_blocks(const FieldArgs& a, bool fast, bool judge = false);
 hipError_t launch_update_e_b(const FieldArgs& a, bool fast, hipStream_t s);
 // E_dyn = E_stat + KE raw_E, B_dyn = B_stat + KMU raw_B for fluid cells (the
 // direct kernel's own epilogue, applied to a.raw).

@@ -21,9 +21,11 @@ namespace ion {
 // ---------------------------------------------------------------------------
 // Source list: LOD indices d in [lo, hi) with a non-zero charge, in index
 // order. A source of zero charge adds exactly zero to every cell, so
-// dropping it leaves all fields unchanged. *mode (if not null): whether the
-// multilevel field update may be used, i.e. there are enough sources and none
-// is infinite, NaN or so large that a partial sum could overflow.
+// dropping it leaves all fields unchanged. mode (if not null): whether the
+// field updates over all LOD blocks may be used, i.e. there are enough sources
+// and none is infinite, NaN or so large that a partial sum could overflow.
+// dense (if not null): (q, v) at every LOD index, whole z layers of the LOD
+// grid, zero where there is no source.
 // ---------------------------------------------------------------------------
 // 4-vectors of the arithmetic type; the 4th component of a source's vd
 // carries its LOD index (float: the bits, double: the value, exact below 2^53).
@@ -52,13 +54,23 @@ __global__ void __launch_bounds__(1024) k_prep_sources(const typename V4F<R>::T*
                                                        uint32_t hi, uint32_t nd, R dsx, R dsy, R dsz,
                                                        typename V4F<R>::T* __restrict__ src_pq,
                                                        typename V4F<R>::T* __restrict__ src_vd,
-                                                       uint32_t* __restrict__ count, uint32_t* __restrict__ mode) {
+                                                       uint32_t* __restrict__ count, uint32_t* __restrict__ mode,
+                                                       float4* __restrict__ dense) {
     __shared__ uint32_t wave_tot[16];
     __shared__ uint32_t base_sh;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6;
     bool wild = false;
     if (tid == 0) base_sh = 0;
     __syncthreads();
+    if constexpr (sizeof(R) == 4) {
+        if (dense != nullptr) {
+            const uint32_t n = (hi + nd * nd - 1) / (nd * nd) * nd * nd;
+            for (uint32_t d = tid; d < n; d += 1024) {
+                const float4 e = d >= lo && d < hi ? qu[d] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                dense[d] = e.x != 0.0f ? e : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+        }
+    }
     for (uint32_t c0 = lo; c0 < hi; c0 += 1024) {
         const uint32_t d = c0 + tid;
         typename V4F<R>::T e = mk4f<R>(R(0), R(0), R(0), R(0));
@@ -95,7 +107,10 @@ __global__ void __launch_bounds__(1024) k_prep_sources(const typename V4F<R>::T*
     const bool any_wild = __syncthreads_or(wild);
     if (tid == 0) {
         *count = base_sh;
-        if (mode != nullptr) *mode = base_sh >= ML_MIN_SOURCES && !any_wild;
+        if (mode != nullptr) {
+            mode[MODE_FAST] = base_sh >= nd * nd * nd / 32 && !any_wild;
+            mode[MODE_EXACT] = base_sh >= nd * nd * nd / 4 && !any_wild;
+        }
     }
 }
 
@@ -119,10 +134,16 @@ __device__ __forceinline__ void interact_exact(R q, R vx, R vy, R vz, R rx, R ry
     bz = bz + q * crz;
 }
 
+// Whether a kernel launched before has done the field update (a.second, and
+// *a.mode says so). No store here: it would keep the compiler from reading the
+// sources as scalars (k_update_e_b_tiled 6 % slower).
+__device__ __forceinline__ bool done_before(const FieldArgs& a) { return a.second != 0u && *a.mode != 0u; }
+
 template <bool FAST, bool NEAR, int CPT>
 __global__ void __launch_bounds__(FIELD_BLOCK) k_update_e_b(FieldArgs a) {
     __shared__ float4 s_pq[FIELD_TILE];
     __shared__ float4 s_vd[FIELD_TILE];
+    if (done_before(a)) return;
     const uint32_t tid = threadIdx.x;
     const uint32_t NX = a.nx, NY = a.ny, NZ = a.nz;
     const uint32_t nd = 1u << a.D;
@@ -307,7 +328,7 @@ __global__ void __launch_bounds__(FIELD_BLOCK) k_update_e_b_f64(FieldArgs a) {
     bd[2 * N + n] = bs[2 * N + n] + kmu * bz;
 }
 
-// The field update on LOD-aligned tiles, EXACT arithmetic. A block covers
+// The field update on LOD-aligned tiles, FAST or EXACT arithmetic. A block covers
 // (ROW*TX) x TY x TZ cells inside one top-level LOD block, so the own-LOD
 // skip is the same for every cell of the block: a wave-uniform branch on the
 // source's LOD index. Each thread owns ROW consecutive cells of one row: the
@@ -325,10 +346,11 @@ __global__ void __launch_bounds__(FIELD_BLOCK) k_update_e_b_f64(FieldArgs a) {
 // Held to 80 VGPRs (6 wavefronts per SIMD, no spills; the sweep's VALU
 // instructions are the same as at 105 VGPRs) so that the scalar loads at the
 // top of each source's iteration hide behind the other wavefronts.
-template <int ROW>
+template <int ROW, bool FAST>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
     __shared__ float s_epi[ROW * 256];
+    if (done_before(a)) return;
     const uint32_t NX = a.nx, NY = a.ny;
     const uint32_t tx = threadIdx.x % TX, ty = (threadIdx.x / TX) % TY, tz = threadIdx.x / (TX * TY);
     const uint32_t tiles_x = NX / (ROW * TX), tiles_y = NY / TY;
@@ -368,7 +390,8 @@ k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
         // arithmetic, so their latency hides behind it
         float4 vd_next = svd[s0], pq_next = spq[s0];
         // one source per iteration: the compiler then lays the ROW cells'
-        // chains side by side
+        // chains side by side (measured at 256^3, FAST: 17.0 ms against
+        // 18.1 ms with two sources per iteration and 17.5 ms with four)
 #pragma unroll 1
         for (uint32_t s = s0; s < s1; s++) {
             const float4 vd = vd_next, pq = pq_next;
@@ -376,24 +399,42 @@ k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
             vd_next = svd[sn];
             pq_next = spq[sn];
             const float ry = py - pq.y, rz = pz - pq.z;
-            // interact_exact with r_y^2, r_z^2 hoisted: pre = r / |r|^3,
-            // e += q pre, b += q (v x pre), every operation rounded on its own
-            const float ry2 = ry * ry, rz2 = rz * rz;
-            const float q = pq.w;
+            if constexpr (FAST) {
+                const float syz = __builtin_fmaf(ry, ry, rz * rz);
+                const float cx = __builtin_fmaf(vd.y, rz, -(vd.z * ry));  // (v x r).x
+                const float m1 = vd.x * rz, m2 = vd.x * ry;
 #pragma unroll
-            for (int k = 0; k < ROW; k++) {
-                const float rx = px[k] - pq.x;
-                const float sm = sqrt_cr((rx * rx + ry2) + rz2);
-                const float cbm = (sm * sm) * sm;
-                const float prx = div_cr(rx, cbm), pry = div_cr(ry, cbm), prz = div_cr(rz, cbm);
-                ex[k] = ex[k] + q * prx;
-                ey[k] = ey[k] + q * pry;
-                ez[k] = ez[k] + q * prz;
-                const float crx = vd.y * prz - vd.z * pry, cry = vd.z * prx - vd.x * prz,
-                            crz = vd.x * pry - vd.y * prx;
-                bxa[k] = bxa[k] + q * crx;
-                bya[k] = bya[k] + q * cry;
-                bza[k] = bza[k] + q * crz;
+                for (int k = 0; k < ROW; k++) {
+                    const float rx = px[k] - pq.x;
+                    const float inv = __builtin_amdgcn_rsqf(__builtin_fmaf(rx, rx, syz));
+                    const float t = pq.w * (inv * inv * inv);
+                    ex[k] = __builtin_fmaf(t, rx, ex[k]);
+                    ey[k] = __builtin_fmaf(t, ry, ey[k]);
+                    ez[k] = __builtin_fmaf(t, rz, ez[k]);
+                    bxa[k] = __builtin_fmaf(t, cx, bxa[k]);
+                    bya[k] = __builtin_fmaf(t, __builtin_fmaf(vd.z, rx, -m1), bya[k]);  // (v x r).y
+                    bza[k] = __builtin_fmaf(t, __builtin_fmaf(-vd.y, rx, m2), bza[k]);  // (v x r).z
+                }
+            } else {
+                // interact_exact with r_y^2, r_z^2 hoisted: pre = r / |r|^3,
+                // e += q pre, b += q (v x pre), every operation rounded on its own
+                const float ry2 = ry * ry, rz2 = rz * rz;
+                const float q = pq.w;
+#pragma unroll
+                for (int k = 0; k < ROW; k++) {
+                    const float rx = px[k] - pq.x;
+                    const float sm = sqrt_cr((rx * rx + ry2) + rz2);
+                    const float cbm = (sm * sm) * sm;
+                    const float prx = div_cr(rx, cbm), pry = div_cr(ry, cbm), prz = div_cr(rz, cbm);
+                    ex[k] = ex[k] + q * prx;
+                    ey[k] = ey[k] + q * pry;
+                    ez[k] = ez[k] + q * prz;
+                    const float crx = vd.y * prz - vd.z * pry, cry = vd.z * prx - vd.x * prz,
+                                crz = vd.x * pry - vd.y * prx;
+                    bxa[k] = bxa[k] + q * crx;
+                    bya[k] = bya[k] + q * cry;
+                    bza[k] = bza[k] + q * crz;
+                }
             }
         }
     };
@@ -450,6 +491,151 @@ k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
         }
     }
     if (a.judge != nullptr) judge_block_sums(jd, a.judge);
+}
+
+// The field update in EXACT arithmetic over all LOD blocks of depth 3 or 4.
+// r / |r|^3 depends on the shift between a cell and a source only, and the
+// cells at one place of their LOD blocks see the sources of every block at the
+// same (2 nd - 1)^3 shifts: its value, rounded as in the reference, is computed
+// once for a shift and read by every pair with that shift. What is left per
+// pair are the 21 unfused multiplications and additions, in the reference's
+// order (ascending LOD index for every cell).
+//
+// A wavefront takes the cells at (ox, oy, oz) of all blocks of a z layer of the
+// LOD grid (depth 3: of four layers), a lane four blocks in a row along x. For
+// each layer of sources it tabulates the shifts in that layer in LDS (an entry
+// serves 64 or so pairs), then goes through the sources, (q, v) as scalar
+// operands: of a row's shifts a lane holds the four of its blocks and the four
+// below, so that four sources cost three 16-byte LDS reads.
+// A source without charge adds +-0 to sums that are never -0; the shift of a
+// block to itself, which the reference leaves out, tabulates as 0 and does the
+// same (sources that are not finite take the kernels above).
+//
+// Bound by VALU issue (4 cycles an instruction): 128^3 with 3511 sources
+// 8.2 -> 3.5 ms (21 x 4 cycles a pair are 3.0 ms), 256^3 57.2 -> 22.7 ms, 176 x 112
+// x 208 (blocks of 11 x 7 x 13 cells) 20.3 -> 6.3 ms. The direct kernels, whose
+// time goes with the number of sources, are used below a quarter of the LOD
+// blocks charged, 1024 of 4096: 128^3 with 819 sources 1.64 ms there and 2.0 here.
+//
+// Workgroups of one (oy, oz, layer) run on one XCD (block b runs on XCD b % 8),
+// ox fastest: their stores, 16 cells apart, meet in its L2.
+template <int ND>
+__global__ void __launch_bounds__(64) k_update_e_b_shifts(FieldArgs a, uint32_t dz0, uint32_t zext, uint32_t blocks0) {
+    constexpr int XG = ND / 4, PL = 64 / (XG * ND), RS = 2 * ND, ROWS = 2 * ND - 1;
+    __shared__ __align__(16) float tab[3][PL][ROWS][RS];
+    const int lane = (int)threadIdx.x;
+    const int bx = (int)(a.nx / ND), by = (int)(a.ny / ND), bz = (int)(a.nz / ND);
+    double* const judge = a.judge == nullptr ? nullptr : a.judge + (size_t)blocks0 * 4;
+    const uint32_t i0 = blockIdx.x / 8u;
+    const int ox = (int)(i0 % (uint32_t)bx), grp = (int)(i0 / (uint32_t)bx) * 8 + (int)(blockIdx.x % 8u);
+    float jd[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int oy = grp % by, oz = grp / by % bz, zb = grp / (by * bz);
+    if (*a.mode != 0u && zb < ND / PL) {
+        const int xg = lane % XG, Y = lane / XG % ND, zs = lane / (XG * ND);
+        const int Z = zb * PL + zs;
+        uint64_t cell[4];
+        bool live[4];
+        float acc[4][6];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            cell[j] = (uint64_t)((4 * xg + j) * bx + ox) + ((uint64_t)(Y * by + oy) + (uint64_t)(Z * bz + oz) * a.ny) * a.nx;
+            live[j] = (a.flags[cell[j]] & 0x1F) != 0x01;
+#pragma unroll
+            for (int c = 0; c < 6; c++) acc[j][c] = 0.0f;
+        }
+        typedef float f32x16 __attribute__((ext_vector_type(16), aligned(4)));
+        typedef const __attribute__((address_space(4))) float* cfloat_p;  // not written by this kernel
+        typedef const __attribute__((address_space(4))) f32x16* cf32x16_p;
+        const cfloat_p src = (cfloat_p)a.dense;
+        // the specialised operators hold for |r|^2 < 2^24 (cr_math.hpp)
+        const bool special = a.nx < 2048u && a.ny < 2048u && zext * (uint32_t)bz < 2048u;
+        if (__any(live[0] || live[1] || live[2] || live[3])) {
+            for (int Dz = (int)dz0; Dz < (int)zext; Dz++) {
+                // a layer without sources (the range ends in some, above the domain)
+                bool some = false;
+#pragma unroll
+                for (int i = 0; i < ND * ND / 64; i++) some |= a.dense[Dz * ND * ND + i * 64 + lane].x != 0.0f;
+                if (!__any(some)) continue;
+                __syncthreads();
+                for (int i = lane; i < PL * ROWS * RS; i += 64) {
+                    const int sx = i % RS - ND, sy = i / RS % ROWS - (ND - 1), p = i / (RS * ROWS), sz = zb * PL + p - Dz;
+                    const float rx = (float)(sx * bx + ox) - 0.5f * (float)bx, ry = (float)(sy * by + oy) - 0.5f * (float)by,
+                                rz = (float)(sz * bz + oz) - 0.5f * (float)bz;
+                    const float r2 = (rx * rx + ry * ry) + rz * rz;
+                    const bool own = (sx | sy | sz) == 0;
+                    float fx, fy, fz;
+                    if (special) {
+                        const float sm = sqrt_cr(own ? 1.0f : r2);
+                        const float cbm = (sm * sm) * sm;
+                        fx = div_cr(rx, cbm);
+                        fy = div_cr(ry, cbm);
+                        fz = div_cr(rz, cbm);
+                    } else {
+                        const float sm = sqrtf(own ? 1.0f : r2);
+                        const float cbm = (sm * sm) * sm;
+                        fx = rx / cbm;
+                        fy = ry / cbm;
+                        fz = rz / cbm;
+                    }
+                    float* const t = &tab[0][0][0][0] + i;
+                    t[0] = own ? 0.0f : fx;
+                    t[PL * ROWS * RS] = own ? 0.0f : fy;
+                    t[2 * PL * ROWS * RS] = own ? 0.0f : fz;
+                }
+                __syncthreads();
+                for (int Dy = 0; Dy < ND; Dy++) {
+                    const float4* const row = (const float4*)&tab[0][zs][Y - Dy + ND - 1][4 * xg + ND];
+                    float4 A[3], B[3];  // shifts 4 xg - D .. + 3 and the four below
+#pragma unroll
+                    for (int c = 0; c < 3; c++) A[c] = row[c * (PL * ROWS * RS / 4)];
+                    const cfloat_p sp = src + 4 * (Dz * ND + Dy) * ND;
+                    f32x16 next = *(const cf32x16_p)sp;
+#pragma unroll
+                    for (int D = 0; D < ND; D += 4) {
+                        const f32x16 s = next;
+                        if (D + 4 < ND) next = *(const cf32x16_p)(sp + 4 * (D + 4));
+#pragma unroll
+                        for (int c = 0; c < 3; c++) B[c] = row[c * (PL * ROWS * RS / 4) - D / 4 - 1];
+                        const uint32_t charged = (__float_as_uint(s[0]) | __float_as_uint(s[4]) | __float_as_uint(s[8]) |
+                                                  __float_as_uint(s[12])) << 1;
+#pragma unroll
+                        for (int k = 0; charged != 0u && k < 4; k++) {
+                            const float q = s[4 * k], vx = s[4 * k + 1], vy = s[4 * k + 2], vz = s[4 * k + 3];
+#pragma unroll
+                            for (int j = 0; j < 4; j++) {
+                                float p[3];
+#pragma unroll
+                                for (int c = 0; c < 3; c++) {
+                                    const float4 w = j >= k ? A[c] : B[c];
+                                    const int e = (j - k) & 3;
+                                    p[c] = e == 0 ? w.x : e == 1 ? w.y : e == 2 ? w.z : w.w;
+                                }
+                                acc[j][0] = acc[j][0] + q * p[0];
+                                acc[j][1] = acc[j][1] + q * p[1];
+                                acc[j][2] = acc[j][2] + q * p[2];
+                                const float crx = vy * p[2] - vz * p[1], cry = vz * p[0] - vx * p[2],
+                                            crz = vx * p[1] - vy * p[0];
+                                acc[j][3] = acc[j][3] + q * crx;
+                                acc[j][4] = acc[j][4] + q * cry;
+                                acc[j][5] = acc[j][5] + q * crz;
+                            }
+                        }
+#pragma unroll
+                        for (int c = 0; c < 3; c++) A[c] = B[c];
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (live[j]) write_cell(a, cell[j], acc[j], jd);
+    }
+    if (judge != nullptr) {
+        judge_block_sums(jd, judge);  // zero if the direct kernel does the update,
+        if (*a.mode != 0u)            // whose own sums are else
+            for (uint32_t i = blockIdx.x; i < blocks0; i += gridDim.x)
+                if (lane < 4) a.judge[(size_t)i * 4 + lane] = 0.0;
+    }
 }
 
 __global__ void k_combine_fields(FieldArgs a) {
@@ -514,15 +700,16 @@ __global__ void __launch_bounds__(256) k_sum_f64(const T* __restrict__ x, const 
 
 hipError_t launch_prep_sources(const void* qu_lod, bool f64, uint32_t lo, uint32_t hi, uint32_t nx, uint32_t ny,
                                uint32_t nz, uint32_t D, void* src_pq, void* src_vd, uint32_t* count, uint32_t* mode,
-                               hipStream_t s) {
+                               float4* dense, hipStream_t s) {
     const uint32_t nd = 1u << D;
     const float dx = (float)(nx / nd), dy = (float)(ny / nd), dz = (float)(nz / nd);
     if (f64)
         hipLaunchKernelGGL(k_prep_sources<double>, dim3(1), dim3(1024), 0, s, (const double4*)qu_lod, lo, hi, nd,
-                           (double)dx, (double)dy, (double)dz, (double4*)src_pq, (double4*)src_vd, count, mode);
+                           (double)dx, (double)dy, (double)dz, (double4*)src_pq, (double4*)src_vd, count, mode,
+                           nullptr);
     else
         hipLaunchKernelGGL(k_prep_sources<float>, dim3(1), dim3(1024), 0, s, (const float4*)qu_lod, lo, hi, nd, dx,
-                           dy, dz, (float4*)src_pq, (float4*)src_vd, count, mode);
+                           dy, dz, (float4*)src_pq, (float4*)src_vd, count, mode, dense);
     return hipGetLastError();
 }
 
@@ -549,34 +736,69 @@ static FieldShape field_shape(const FieldArgs& a, bool fast) {
     return FieldShape{0, 0, 0, 0, (uint32_t)((a.N + per - 1) / per)};
 }
 
-uint32_t field_blocks(const FieldArgs& a, bool fast) {
-    MlArgs m;
-    if (fast && ml_plan(a, &m)) return ml_blocks(m);
-    return field_shape(a, fast).blocks;
+// The shift kernel: EXACT arithmetic at LOD depth 3 and 4 without a near
+// field. Workgroups of a z layer's (oy, oz), rounded up to the 8 XCDs.
+static uint32_t shift_blocks(const FieldArgs& a) {
+    if (a.f64 || a.near || (a.D != 3 && a.D != 4) || a.mode == nullptr || a.dense == nullptr) return 0;
+    const uint32_t nd = 1u << a.D, groups = (a.ny / nd) * (a.nz / nd) * (a.D == 4 ? 16u : 2u);
+    return (groups + 7) / 8 * 8 * (a.nx / nd);
 }
 
-hipError_t launch_update_e_b(const FieldArgs& a, bool fast, hipStream_t s) {
+uint32_t field_blocks(const FieldArgs& a, bool fast) {
+    return field_shape(a, fast).blocks + (fast ? 0 : shift_blocks(a));
+}
+
+bool over_all_blocks(const FieldArgs& a, bool fast, bool judge) {
+    MlArgs m;
+    return fast ? !judge && a.judge == nullptr && a.raw == nullptr && ml_plan(a, &m) : shift_blocks(a) != 0;
+}
+
+// The update over all LOD blocks first, where there is one (FAST: not for the
+// surrogate's judge and training target, which stay the plain sum), then a
+// direct kernel; *a.mode says which of the two does the work.
+hipError_t launch_update_e_b(const FieldArgs& args, bool fast, hipStream_t s) {
     constexpr int CPT_EXACT = 1, CPT_FAST = 2;
-    if (fast && !a.f64 && !a.near) {
-        MlArgs m;
-        return ml_plan(a, &m) ? launch_field_fast(m, s) : hipErrorInvalidValue;
-    }
+    FieldArgs a = args;
+    a.second = 0;
     const FieldShape sh = field_shape(a, fast);
     if (a.f64) {
         if (a.judge != nullptr) return hipErrorInvalidValue;
         hipLaunchKernelGGL(k_update_e_b_f64, dim3(sh.blocks), dim3(FIELD_BLOCK), 0, s, a);
         return hipGetLastError();
     }
+    MlArgs m;
+    if (fast && a.judge == nullptr && a.raw == nullptr && ml_plan(a, &m)) {
+        const hipError_t e = launch_field_fast(m, s);
+        if (e != hipSuccess) return e;
+        a.second = 1;
+        a.mode = args.mode + MODE_FAST;
+    }
+    if (const uint32_t nb = fast ? 0 : shift_blocks(a)) {
+        const uint32_t nd = 1u << a.D;
+        uint32_t n_lod = 0;
+        for (uint32_t i = 0; i <= a.D; i++) n_lod += 1u << (3 * i);
+        a.mode = args.mode + MODE_EXACT;
+        const uint32_t dz0 = (n_lod - nd * nd * nd) / (nd * nd), zext = (n_lod + nd * nd - 1) / (nd * nd);
+        if (a.D == 4) hipLaunchKernelGGL(k_update_e_b_shifts<16>, dim3(nb), dim3(64), 0, s, a, dz0, zext, sh.blocks);
+        else hipLaunchKernelGGL(k_update_e_b_shifts<8>, dim3(nb), dim3(64), 0, s, a, dz0, zext, sh.blocks);
+        a.second = 1;
+    }
     if (sh.row) {
         const uint32_t TX = sh.TX, TY = sh.TY, TZ = sh.TZ;
         const dim3 g(sh.blocks), bl(TX * TY * TZ);
-        if (sh.row == 8) hipLaunchKernelGGL((k_update_e_b_tiled<8>), g, bl, 0, s, a, TX, TY, TZ);
-        else hipLaunchKernelGGL((k_update_e_b_tiled<4>), g, bl, 0, s, a, TX, TY, TZ);
+        if (fast) {
+            if (sh.row == 8) hipLaunchKernelGGL((k_update_e_b_tiled<8, true>), g, bl, 0, s, a, TX, TY, TZ);
+            else hipLaunchKernelGGL((k_update_e_b_tiled<4, true>), g, bl, 0, s, a, TX, TY, TZ);
+        } else {
+            if (sh.row == 8) hipLaunchKernelGGL((k_update_e_b_tiled<8, false>), g, bl, 0, s, a, TX, TY, TZ);
+            else hipLaunchKernelGGL((k_update_e_b_tiled<4, false>), g, bl, 0, s, a, TX, TY, TZ);
+        }
         return hipGetLastError();
     }
     const dim3 g(sh.blocks), b(FIELD_BLOCK);
     if (fast) {
-        hipLaunchKernelGGL((k_update_e_b<true, true, CPT_FAST>), g, b, 0, s, a);
+        if (a.near) hipLaunchKernelGGL((k_update_e_b<true, true, CPT_FAST>), g, b, 0, s, a);
+        else hipLaunchKernelGGL((k_update_e_b<true, false, CPT_FAST>), g, b, 0, s, a);
     } else {
         if (a.near) hipLaunchKernelGGL((k_update_e_b<false, true, CPT_EXACT>), g, b, 0, s, a);
         else hipLaunchKernelGGL((k_update_e_b<false, false, CPT_EXACT>), g, b, 0, s, a);

@@ -247,14 +247,19 @@ ion::LbmArgs lbm_args(ion_handle* h) {
     return a;
 }
 
+// The dense LOD sources of a multilevel workspace (depth 3 and 4), or null.
+float4* ml_dense(float* ws, uint32_t D) { return ws && (D == 3 || D == 4) ? (float4*)(ws + ion::ML_DENSE) : nullptr; }
+
 // update_e_b_dynamic for the current buffers (sim_kernels.cl:897-993).
-// Compacted LOD sources (q != 0) of the range update_e_b_dynamic reads.
-int prep_sources(ion_handle* h) {
+// Compacted LOD sources (q != 0) of the range update_e_b_dynamic reads; all:
+// also what the updates over all LOD blocks need.
+int prep_sources(ion_handle* h, bool all) {
     const uint64_t n_top = (uint64_t)h->nd * h->nd * h->nd;
     const uint32_t hi = (uint32_t)h->n_lod, lo = (uint32_t)(h->n_lod - n_top);
     return timed(h, 2, [&] {
         return ion::launch_prep_sources(h->qu_lod, h->f64(), lo, hi, h->cfg.n_x, h->cfg.n_y, h->cfg.n_z, h->D,
-                                        h->src_pq, h->src_vd, h->src_count, (uint32_t*)h->ml_ws, h->stream);
+                                        h->src_pq, h->src_vd, h->src_count, all ? (uint32_t*)h->ml_ws : nullptr,
+                                        all ? ml_dense(h->ml_ws, h->D) : nullptr, h->stream);
     });
 }
 
@@ -289,13 +294,15 @@ ion::FieldArgs field_args(ion_handle* h) {
     f.f64 = h->f64() ? 1u : 0u;
     f.qu = (const float4*)h->qu_lod;
     f.ml_ws = h->ml_ws;
+    f.mode = (const uint32_t*)h->ml_ws;
+    f.dense = ml_dense(h->ml_ws, h->D);
     return f;
 }
 
 int field_update(ion_handle* h) {
-    int rc = prep_sources(h);
-    if (rc) return rc;
     const ion::FieldArgs f = field_args(h);
+    int rc = prep_sources(h, ion::over_all_blocks(f, h->field_mode == ION_FIELD_FAST));
+    if (rc) return rc;
     return timed(h, 3, [&] {
         hipError_t e = ion::launch_update_e_b(f, h->field_mode == ION_FIELD_FAST, h->stream);
         if (e == hipSuccess && f.raw != nullptr) e = ion::launch_combine_fields(f, h->stream);
@@ -315,11 +322,11 @@ ion::sur::Fields sur_fields(ion_handle* h) {
 // so no 6 x N buffer is needed for either. Residuals: relative L2 of the
 // dynamic E and B over the fluid cells.
 int judged_field_update(ion_handle* h, double* rel_e, double* rel_b) {
-    int rc = prep_sources(h);
-    if (rc) return rc;
     ion::FieldArgs f = field_args(h);
     f.raw = nullptr;
     const bool fast = h->field_mode == ION_FIELD_FAST;
+    int rc = prep_sources(h, ion::over_all_blocks(f, fast, true));
+    if (rc) return rc;
     if (!h->judge_partials) {
         const uint32_t nb = std::max(ion::field_blocks(f, true), ion::field_blocks(f, false));
         if ((rc = dalloc(h, (void**)&h->judge_partials, ((size_t)nb + 1) * 4 * sizeof(double)))) return rc;
@@ -368,7 +375,7 @@ int field_step(ion_handle* h) {
         }
         return ION_OK;
     }
-    if ((rc = prep_sources(h))) return rc;
+    if ((rc = prep_sources(h, false))) return rc;
     bool ok = true;
     rc = timed(h, 3, [&] {
         ok = h->net->infer(sur_fields(h)) == 0;
@@ -598,11 +605,14 @@ int ion_create(const ion_config* cfg, ion_handle** out) {
         if ((rc = dalloc(h, (void**)&h->q, N * rs))) return bail(rc);
         if ((rc = dalloc(h, (void**)&h->qu_lod, h->n_lod * 4 * rs))) return bail(rc);
         const uint64_t n_top = (uint64_t)h->nd * h->nd * h->nd;
-        if ((rc = dalloc(h, (void**)&h->src_pq, n_top * 4 * rs))) return bail(rc);
-        if ((rc = dalloc(h, (void**)&h->src_vd, n_top * 4 * rs))) return bail(rc);
-        if ((rc = dalloc(h, (void**)&h->src_count, sizeof(uint32_t)))) return bail(rc);
-        ion::MlArgs ml;
-        if (ion::ml_plan(field_args(h), &ml) && (rc = dalloc(h, (void**)&h->ml_ws, ml.ws_floats * sizeof(float)))) return bail(rc);
+        // the field update's sources and workspace, in one allocation
+        const size_t src_b = n_top * 4 * rs, count_b = 256;
+        char* work = nullptr;
+        if ((rc = dalloc(h, (void**)&work, 2 * src_b + count_b + ion::ml_workspace(field_args(h)) * sizeof(float)))) return bail(rc);
+        h->src_pq = (float4*)work;
+        h->src_vd = (float4*)(work + src_b);
+        h->src_count = (uint32_t*)(work + 2 * src_b);
+        if (ion::ml_workspace(field_args(h))) h->ml_ws = (float*)(work + 2 * src_b + count_b);
         if (h->lod && (rc = dalloc(h, (void**)&h->lod_seg, (N / h->lod_bx) * 4 * rs))) return bail(rc);
         h->ecr = cfg->ext_subgrid_ecr != 0;
         if (h->ecr) {
@@ -945,7 +955,7 @@ int ion_update_e_b_noalloc(const ion_config* cfg, const ion_field_buffers* b, in
     float* ml_ws = (float*)(s + 2 * ION_NOALLOC_MAX_SOURCES + 16);
     hipStream_t st = (hipStream_t)stream;
     hipError_t e = ion::launch_prep_sources(b->qu_lod, false, lo, hi, cfg->n_x, cfg->n_y, cfg->n_z, D, src_pq, src_vd,
-                                            count, (uint32_t*)ml_ws, st);
+                                            count, (uint32_t*)ml_ws, ml_dense(ml_ws, D), st);
     if (e != hipSuccess) return fail(ION_ERR_DEVICE, std::string("source compaction: ") + hipGetErrorString(e));
     f.e_stat = b->e_stat;
     f.b_stat = b->b_stat;
@@ -968,6 +978,8 @@ int ion_update_e_b_noalloc(const ion_config* cfg, const ion_field_buffers* b, in
     f.f64 = 0u;
     f.qu = (const float4*)b->qu_lod;
     f.ml_ws = ml_ws;
+    f.mode = (const uint32_t*)ml_ws;
+    f.dense = ml_dense(ml_ws, D);
     e = ion::launch_update_e_b(f, field_mode == ION_FIELD_FAST, st);
     if (e != hipSuccess) return fail(ION_ERR_DEVICE, std::string("field kernel: ") + hipGetErrorString(e));
     return ION_OK;
@@ -981,7 +993,7 @@ static int need_net(ion_handle* h) {
 
 int ion_surrogate_infer(ion_handle* h) {
     int rc = need_net(h);
-    if (rc || (rc = prep_sources(h))) return rc;
+    if (rc || (rc = prep_sources(h, false))) return rc;
     bool ok = true;
     rc = timed(h, 3, [&] {
         ok = h->net->infer(sur_fields(h)) == 0;
@@ -995,7 +1007,7 @@ int ion_surrogate_infer(ion_handle* h) {
 
 int ion_surrogate_train_step(ion_handle* h, int update, double* rel_e, double* rel_b) {
     int rc = need_net(h);
-    if (rc || (rc = prep_sources(h))) return rc;
+    if (rc || (rc = prep_sources(h, false))) return rc;
     double re = 0, rb = 0;
     if (h->net->train_step(sur_fields(h), update != 0, &re, &rb)) return fail(ION_ERR_DEVICE, "surrogate: " + h->net->error());
     HIPCHK(hipStreamSynchronize(h->stream));
@@ -1007,7 +1019,7 @@ int ion_surrogate_train_step(ion_handle* h, int update, double* rel_e, double* r
 
 int ion_surrogate_residual(ion_handle* h, double* rel_e, double* rel_b) {
     int rc = need_net(h);
-    if (rc || (rc = prep_sources(h))) return rc;
+    if (rc || (rc = prep_sources(h, false))) return rc;
     double re = 0, rb = 0;
     if (h->net->residual(sur_fields(h), &re, &rb)) return fail(ION_ERR_DEVICE, "surrogate: " + h->net->error());
     if (rel_e) *rel_e = re;
