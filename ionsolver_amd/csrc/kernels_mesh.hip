@@ -355,6 +355,262 @@ __global__ __launch_bounds__(FLD_BLOCK) void k_static_e(Sources src, const uint8
     E[2 * N + n] += ez * ke;
 }
 
+// ---------------------------------------------------------------------------
+// Both sums by shifts. A mesh has one magnetisation (charge) for all its cells,
+// so what a source adds depends only on the shift between it and the target.
+// The sources are grouped in aligned fours along x, and these in batches of one
+// value, one z layer and a window of rows and columns (SHIFT_ROWS x
+// BATCH_COLS). A workgroup takes SHIFT_ROWS target rows of up to TILE_Q aligned fours
+// in a z layer; for each batch it tabulates the contribution of every shift
+// that occurs, with the arithmetic of the kernels above, and adds the entries
+// up in the reference's order: one addition per target, source and component
+// instead of 36 (psi) or some 90 instructions. A lane holds four targets; the
+// shifts of four sources to them are two aligned fours of a table row.
+// A source's own cell tabulates as 0: the sums start at +0 and are never -0.
+// The kernels above are bound by the vector units' square roots and divisions;
+// this one by the table loads' latency and the scalar work of a group, beside
+// its additions (0.7 ms below). Ring and box of solid cells in 96^3, us: psi
+// 24900 -> 3630, E 16000 -> 1730; the call of both, copies included, 43.1 ->
+// 8.5 ms. Bit-identical.
+// ---------------------------------------------------------------------------
+constexpr int BATCH_COLS = 128, TILE_Q = 32;
+template <int NC> constexpr int SHIFT_ROWS = NC == 1 ? 16 : 8;  // rows of a batch, and target rows of a workgroup
+constexpr int GRP_THREADS = 1024;
+constexpr int TAB_ROW = TILE_Q + BATCH_COLS / 4;  // aligned fours of a table row
+
+__device__ __forceinline__ bool same_value(float4 a, float4 b) {
+    return __float_as_uint(a.x) == __float_as_uint(b.x) && __float_as_uint(a.y) == __float_as_uint(b.y) &&
+           __float_as_uint(a.z) == __float_as_uint(b.z);
+}
+
+// Groups and batches of the sources (in ascending cell order), by one
+// workgroup. counts: groups, batches.
+__global__ __launch_bounds__(GRP_THREADS) void k_group(Sources src, ShiftLists out, int rows) {
+    __shared__ uint32_t wg[GRP_THREADS / 64], wb[GRP_THREADS / 64];
+    __shared__ int wr[GRP_THREADS / 64];  // first row of the last run that begins in a wavefront, or -1
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wv = tid >> 6, n = src.count[0];
+    const uint64_t below = (1ull << lane) - 1ull;
+    uint32_t ng = 0, nb = 0;
+    int carry = -1;  // the same of the sources before
+    for (uint32_t base = 0; base < n; base += GRP_THREADS) {
+        const uint32_t i = base + tid;
+        bool g = false, b = false, run = false;
+        float4 p = make_float4(0.0f, 0.0f, 0.0f, 0.0f), v = p, q = p;
+        int x = 0, y = 0;
+        if (i < n) {
+            p = src.pos[i];
+            v = src.val[i];
+            x = (int)p.x;
+            y = (int)p.y;
+            g = b = run = true;
+            if (i > 0) {
+                q = src.pos[i - 1];
+                run = !same_value(v, src.val[i - 1]) || q.z != p.z;
+                g = run || (int)q.x >> 2 != x >> 2 || (int)q.y != y;
+            }
+        }
+        // first row of the run the source before belongs to
+        const uint64_t mr = __ballot(run), before = mr & below;
+        const int own_first = __shfl(y, before ? 63 - __builtin_clzll(before) : 0);
+        const int last_y = __shfl(y, mr ? 63 - __builtin_clzll(mr) : 0);
+        __syncthreads();
+        if (lane == 0) wr[wv] = mr ? last_y : -1;
+        __syncthreads();
+        int y0 = carry;
+        for (uint32_t w = 0; w < GRP_THREADS / 64; w++) {
+            if (w < wv && wr[w] >= 0) y0 = wr[w];
+            if (wr[w] >= 0) carry = wr[w];
+        }
+        if (before) y0 = own_first;
+        if (run) y0 = y;
+        b = i < n;
+        if (i < n && !run)
+            b = ((int)q.y - y0) / rows != (y - y0) / rows || (int)q.x / BATCH_COLS != x / BATCH_COLS;
+        g = g || b;
+        const uint64_t mg = __ballot(g), mb = __ballot(b);
+        __syncthreads();
+        if (lane == 0) {
+            wg[wv] = (uint32_t)__popcll(mg);
+            wb[wv] = (uint32_t)__popcll(mb);
+        }
+        __syncthreads();
+        uint32_t og = ng + (uint32_t)__popcll(mg & below), ob = nb + (uint32_t)__popcll(mb & below);
+        for (uint32_t w = 0; w < GRP_THREADS / 64; w++) {
+            if (w < wv) {
+                og += wg[w];
+                ob += wb[w];
+            }
+            ng += wg[w];
+            nb += wb[w];
+        }
+        if (g) {
+            uint32_t mask = 1u << (x & 3);
+            for (uint32_t k = i + 1; k < n && k < i + 4; k++) {
+                const float4 q = src.pos[k];
+                if (!same_value(v, src.val[k]) || (int)q.x >> 2 != x >> 2 || (int)q.y != y || q.z != p.z) break;
+                mask |= 1u << ((int)q.x & 3);
+            }
+            const int rel = (y - y0) % rows * TAB_ROW + (x % BATCH_COLS >> 2);
+            out.groups[og] = (uint32_t)rel << 4 | mask;
+        }
+        if (b) {
+            out.first[ob] = og;
+            out.val[ob] = make_float4(v.x, v.y, v.z, p.z);
+            out.origin[ob] = make_int2(x / BATCH_COLS * (BATCH_COLS / 4), y0 + (y - y0) / rows * rows);
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        out.first[nb] = ng;
+        out.counts[0] = ng;
+        out.counts[1] = nb;
+    }
+}
+
+// NC = 1: psi of the padded lattice; NC = 3: E.
+// First and last column of fours of each batch, one batch a wavefront.
+__global__ __launch_bounds__(64) void k_batch_cols(ShiftLists l) {
+    const uint32_t b = blockIdx.x, g1 = l.first[b + 1], xw = (uint32_t)l.origin[b].x;
+    uint32_t lo = TAB_ROW, hi = 0;
+    for (uint32_t g = l.first[b] + threadIdx.x; g < g1; g += 64) {
+        const uint32_t x = (l.groups[g] >> 4) % TAB_ROW;
+        lo = min(lo, x);
+        hi = max(hi, x);
+    }
+    for (int d = 32; d > 0; d >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, d));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, d));
+    }
+    if (threadIdx.x == 0) l.cols[b] = make_int2((int)(xw + lo), (int)(xw + hi));
+}
+
+template <int NC>
+__global__ __launch_bounds__(512) void k_shift_sums(Sources src, ShiftLists list, const uint8_t* flags, float* out, uint32_t nx,
+                                                    uint32_t ny, uint32_t nz, float ke, uint32_t tile_q) {
+    constexpr int ROWS = SHIFT_ROWS<NC>;
+    constexpr int TAB = (2 * ROWS - 1) * TAB_ROW;
+    __shared__ float4 tab[NC][TAB];
+    const uint32_t TX = NC == 1 ? nx + 2u : nx, TY = NC == 1 ? ny + 2u : ny;  // targets
+    const int tid = (int)threadIdx.x, T = (int)blockDim.x;
+    const int Q = (int)tile_q, q = tid % Q, r = tid / Q;
+    const int q0 = (int)blockIdx.x * Q, y0 = (int)blockIdx.y * ROWS, z = (int)blockIdx.z;
+    const bool special = NC == 1 && src.count[1] == 0u && nx + 2u < 2048u && ny + 2u < 2048u && nz + 2u < 2048u;
+    typedef const __attribute__((address_space(4))) uint32_t* cuint_p;  // not written by this kernel
+    const cuint_p first = (cuint_p)list.first, groups = (cuint_p)list.groups, vals = (cuint_p)(const uint32_t*)list.val,
+                  cols = (cuint_p)(const uint32_t*)list.cols, origin = (cuint_p)(const uint32_t*)list.origin;
+    const float4* const mine = &tab[0][0] + (r < ROWS ? r : 0) * TAB_ROW + q;
+    float acc[4][NC];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int c = 0; c < NC; c++) acc[j][c] = 0.0f;
+    for (uint32_t b = 0; b < list.nbatch; b++) {
+        const uint32_t g0 = first[b], g1 = first[b + 1];
+        const float vx = __uint_as_float(vals[4 * b]), vy = __uint_as_float(vals[4 * b + 1]), vz = __uint_as_float(vals[4 * b + 2]);
+        const int sz = (int)__uint_as_float(vals[4 * b + 3]);
+        const int xq0 = (int)cols[2 * b], xq1 = (int)cols[2 * b + 1], xw = (int)origin[2 * b];
+        const int last_rel = (int)(groups[g1 - 1] >> 4) / TAB_ROW;         // the batch's last row, from
+        const int ys1 = (int)origin[2 * b + 1] + last_rel;                 // its window's first
+        const int rows = ROWS + last_rel - (int)(groups[g0] >> 4) / TAB_ROW;
+        // row w of the table: target row y0 + r against source row ys, w = r + ys1 - ys;
+        // entry e: target x - source x = e + 4 (q0 - xq1 - 1)
+        const int W = 4 * (Q + xq1 - xq0 + 1);
+        const float dz = (float)z - (float)sz, inv_w = 1.0f / (float)W;
+        __syncthreads();  // the last batch's table is read
+        for (int i = tid; i < rows * W; i += T) {
+            const int w = (int)(((float)i + 0.5f) * inv_w), e = i - w * W;  // i < 2^13: exact
+            const float dx = (float)(e + 4 * (q0 - xq1 - 1)), dy = (float)(y0 - ys1 + w);
+            const float l2 = dx * dx + dy * dy + dz * dz;
+            float* const t = (float*)&tab[0][w * TAB_ROW] + e;
+            if constexpr (NC == 1) {
+                const float d = dx * vx + dy * vy + dz * vz;
+                float p;
+                if (special) {
+                    const float l = sqrt_cr(l2);
+                    p = div_cr(d, l * l * l);
+                } else {
+                    const float l = sqrtf(l2);
+                    p = d / (l * l * l);
+                }
+                *t = l2 != 0.0f ? p : 0.0f;
+            } else {
+                const float l = sqrtf(l2);
+                const float c3 = l * l * l;
+                t[0] = l2 != 0.0f ? dx * vx / c3 : 0.0f;
+                t[4 * TAB] = l2 != 0.0f ? dy * vx / c3 : 0.0f;
+                t[8 * TAB] = l2 != 0.0f ? dz * vx / c3 : 0.0f;
+            }
+        }
+        __syncthreads();
+        // place of a group's shifts: (ys1 - ys) TAB_ROW + xq1 - xq + 1
+        const int at0 = last_rel * TAB_ROW + (xq1 - xw) + 1;
+        float4 A[NC], B[NC];
+        auto add = [&](int k) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int c = 0; c < NC; c++) {
+                    const float4 w = j >= k ? A[c] : B[c];
+                    const int e = (j - k) & 3;
+                    acc[j][c] += e == 0 ? w.x : e == 1 ? w.y : e == 2 ? w.z : w.w;
+                }
+        };
+        uint32_t next = groups[g0];
+        int last = -1;
+        for (uint32_t g = g0; g < g1; g++) {
+            const uint32_t word = next, mask = word & 15u;
+            next = groups[g + 1 < g1 ? g + 1 : g];
+            const int at = at0 - (int)(word >> 4);
+            if (at != last) {  // a group to the right of the last one goes one four down
+#pragma unroll
+                for (int c = 0; c < NC; c++) B[c] = mine[c * TAB + at];
+            }
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                A[c] = B[c];
+                B[c] = mine[c * TAB + at - 1];
+            }
+            last = at - 1;
+            if (mask == 15u) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) add(k);
+            } else {
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (mask >> k & 1u) add(k);
+            }
+        }
+    }
+    const uint32_t y = (uint32_t)(y0 + r);
+    if (r >= ROWS || y >= TY) return;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t x = 4u * (uint32_t)(q0 + q) + (uint32_t)j;
+        if (x >= TX) continue;
+        const uint64_t n = (uint64_t)x + ((uint64_t)y + (uint64_t)z * TY) * TX;
+        if constexpr (NC == 1) {
+            // psic / (4.0f * M_PI): M_PI is a double constant, so the quotient is taken in double
+            out[n] = (float)((double)acc[j][0] / (4.0 * 3.14159265358979323846));
+        } else {
+            const uint64_t N = (uint64_t)nx * ny * nz;
+            if ((flags[n] & TYPE_S) == TYPE_S) continue;
+#pragma unroll
+            for (int c = 0; c < NC; c++) out[c * N + n] += acc[j][c] * ke;
+        }
+    }
+}
+
+template <int NC>
+hipError_t shift_sums(const Sources& src, const ShiftLists& l, const uint8_t* flags, float* out, uint32_t nx,
+                      uint32_t ny, uint32_t nz, float ke, hipStream_t s) {
+    constexpr uint32_t ROWS = SHIFT_ROWS<NC>, pad = NC == 1 ? 2 : 0;
+    const uint32_t quads = (nx + pad + 3) / 4, tiles = (quads + TILE_Q - 1) / TILE_Q, Q = (quads + tiles - 1) / tiles;
+    const dim3 g(tiles, (ny + pad + ROWS - 1) / ROWS, nz + pad), b((Q * ROWS + 63) / 64 * 64);
+    hipLaunchKernelGGL(k_batch_cols, dim3(l.nbatch), dim3(64), 0, s, l);
+    hipLaunchKernelGGL(k_shift_sums<NC>, g, b, 0, s, src, l, flags, out, nx, ny, nz, ke, Q);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 hipError_t launch_voxelize(const VoxArgs& a, hipStream_t s) {
@@ -429,7 +685,34 @@ hipError_t run_psi_math_check(uint64_t* sqrt_mismatch, uint64_t* div_mismatch, u
     return e;
 }
 
-hipError_t launch_psi(const Sources& src, float* psi, uint32_t nx, uint32_t ny, uint32_t nz, hipStream_t s) {
+hipError_t launch_group(int mode, const Sources& src, const ShiftLists& out, hipStream_t s) {
+    hipLaunchKernelGGL(k_group, dim3(1), dim3(GRP_THREADS), 0, s, src, out, mode == 0 ? SHIFT_ROWS<1> : SHIFT_ROWS<3>);
+    return hipGetLastError();
+}
+
+// By shifts or source by source. Of a lattice of N cells with n sources, us,
+// source by source against by shifts (psi | E):
+//   96^3 ring of solid cells, n = 68256   45481 /  7113 | 95996 / 12241
+//   48^3 the same, n = 8544                1031 /   669 |  2512 /  1001
+//   32^3 the same, n = 2496                 281 /   308 |   643 /   404
+//   96^3 each cell with p = 0.3          176884 / 66849 | 370729 / 103323
+//   64^3 the same                         19340 / 13663 |  37013 /  16565
+//   48^3 the same                          3772 /  5376 |   9607 /   7640
+//   64^3 each cell with p = 0.03           1934 /  2690 |   3640 /   3984
+// Few targets leave the chip idle, and a group then costs its latency: it pays
+// if it holds most of its four. A batch's table has to serve enough sources.
+// Grouping itself takes some 40 us with its copy back, and 6 us more for each
+// 1024 sources, against 200 us of direct sums at the least (n N = 2^28).
+bool shifts_possible(uint32_t n, uint64_t N) { return N >= (1u << 16) && n * N >= (1ull << 28); }
+static bool by_shifts(uint32_t n, const ShiftLists& l, uint32_t nx, uint32_t ny, uint32_t nz) {
+    const uint64_t N = (uint64_t)nx * ny * nz;
+    return l.ngroup > 0 && n / l.nbatch >= 48u && (N >= (1u << 18) || n / 2u >= l.ngroup) && nx < (1u << 23) && ny < (1u << 18) &&
+           nz + 2u < 65536u;
+}
+
+hipError_t launch_psi(const Sources& src, uint32_t n, const ShiftLists& l, float* psi, uint32_t nx, uint32_t ny,
+                      uint32_t nz, hipStream_t s) {
+    if (by_shifts(n, l, nx, ny, nz)) return shift_sums<1>(src, l, nullptr, psi, nx, ny, nz, 0.0f, s);
     const uint32_t Np = (nx + 2u) * (ny + 2u) * (nz + 2u);
     hipLaunchKernelGGL(k_psi, dim3((Np + FLD_BLOCK - 1) / FLD_BLOCK), dim3(FLD_BLOCK), 0, s, src, psi, nx, ny, nz);
     return hipGetLastError();
@@ -443,8 +726,9 @@ hipError_t launch_static_b(const uint8_t* flags, float* b, const float* psi, uin
     return hipGetLastError();
 }
 
-hipError_t launch_static_e(const Sources& src, const uint8_t* flags, float* e, uint32_t nx, uint32_t ny, uint32_t nz,
-                           float ke, hipStream_t s) {
+hipError_t launch_static_e(const Sources& src, uint32_t n, const ShiftLists& l, const uint8_t* flags, float* e,
+                           uint32_t nx, uint32_t ny, uint32_t nz, float ke, hipStream_t s) {
+    if (by_shifts(n, l, nx, ny, nz)) return shift_sums<3>(src, l, flags, e, nx, ny, nz, ke, s);
     const uint64_t N = (uint64_t)nx * ny * nz;
     hipLaunchKernelGGL(k_static_e, dim3((uint32_t)((N + FLD_BLOCK - 1) / FLD_BLOCK)), dim3(FLD_BLOCK), 0, s, src,
                        flags, e, nx, ny, nz, ke);

@@ -46,6 +46,19 @@ struct Sources {
     uint32_t* count;
 };
 
+// The sources in aligned fours along x (groups: place in the batch's window,
+// mask of the cells present) and batches of them that share a value, a z layer
+// and a window of rows and columns. Sizes: n each for n sources, first n + 1.
+struct ShiftLists {
+    uint32_t* groups;  // place << 4 | mask
+    float4* val;       // batch: value, z
+    int2* cols;        // batch: first and last x / 4
+    int2* origin;      // batch: window's first x / 4 and row
+    uint32_t* first;   // batch: first group; then the number of groups
+    uint32_t* counts;  // groups, batches
+    uint32_t ngroup, nbatch;  // read back; 0: not grouped
+};
+
 hipError_t launch_voxelize(const VoxArgs& a, hipStream_t s);
 
 // Source selection in two passes, the host reading the total in between:
@@ -63,16 +76,22 @@ hipError_t launch_select_scatter(int mode, const uint8_t* flags, const float* m,
 // square root and division of k_psi against the compiler's general ones.
 hipError_t run_psi_math_check(uint64_t* sqrt_mismatch, uint64_t* div_mismatch, uint64_t* div_samples);
 
+// Groups and batches of the sources (mode as in the selection), where the sums
+// of n sources may be by shifts; their numbers go to out.counts.
+bool shifts_possible(uint32_t n, uint64_t N);
+hipError_t launch_group(int mode, const Sources& src, const ShiftLists& out, hipStream_t s);
+
 // psi over the lattice padded by one cell on every side
 // ((nx+2)(ny+2)(nz+2) values), from the magnet sources.
-hipError_t launch_psi(const Sources& src, float* psi, uint32_t nx, uint32_t ny, uint32_t nz, hipStream_t s);
+hipError_t launch_psi(const Sources& src, uint32_t n, const ShiftLists& l, float* psi, uint32_t nx, uint32_t ny,
+                      uint32_t nz, hipStream_t s);
 // B += -kmu0 grad(psi) (central differences) for cells without the solid bit.
 hipError_t launch_static_b(const uint8_t* flags, float* b, const float* psi, uint32_t nx, uint32_t ny, uint32_t nz,
                            float kmu0, hipStream_t s);
 // E += ke * sum over charged cells of (c - c_i) q_i / |c - c_i|^3, for cells
 // without the solid bit.
-hipError_t launch_static_e(const Sources& src, const uint8_t* flags, float* e, uint32_t nx, uint32_t ny, uint32_t nz,
-                           float ke, hipStream_t s);
+hipError_t launch_static_e(const Sources& src, uint32_t n, const ShiftLists& l, const uint8_t* flags, float* e,
+                           uint32_t nx, uint32_t ny, uint32_t nz, float ke, hipStream_t s);
 
 }  // namespace mesh
 }  // namespace ion

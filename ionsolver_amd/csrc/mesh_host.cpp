@@ -185,34 +185,44 @@ int get_mesh(ion_handle* h, uint32_t index, HandleView* v, const Mesh** m) {
     return ION_OK;
 }
 
-// Sources of one kind compacted on the device; freed by the destructor.
+// Sources of one kind compacted on the device, and their groups; freed by the
+// destructor.
 struct SourceList {
-    uint32_t* counts = nullptr;  // block offsets + total
-    uint32_t* total = nullptr;
-    float4* pos = nullptr;
-    float4* val = nullptr;
+    uint32_t* counts = nullptr;  // block offsets, then count, magnetisation-range flag, groups, batches
+    char* data = nullptr;
     uint32_t n = 0;
+    mesh::Sources src{};
+    mesh::ShiftLists shifts{};
     ~SourceList() {
         (void)hipFree(counts);
-        (void)hipFree(total);
-        (void)hipFree(pos);
-        (void)hipFree(val);
+        (void)hipFree(data);
     }
 };
 
 int select_sources(const HandleView& v, int mode, SourceList* L) {
     const uint32_t nb = mesh::select_blocks(v.N);
-    HIPCHK(hipMalloc((void**)&L->counts, (size_t)(nb + 1) * 4));
-    HIPCHK(hipMalloc((void**)&L->total, 8));  // count, magnetisation-range flag
-    HIPCHK(hipMemsetAsync(L->total, 0, 8, v.stream));
-    HIPCHK(mesh::launch_select_count(mode, v.flags, v.N, L->counts, L->total, v.stream));
-    HIPCHK(hipMemcpyAsync(&L->n, L->total, 4, hipMemcpyDeviceToHost, v.stream));
+    HIPCHK(hipMalloc((void**)&L->counts, (size_t)(nb + 5) * 4));
+    uint32_t* const total = L->counts + nb + 1;
+    HIPCHK(hipMemsetAsync(total, 0, 16, v.stream));
+    HIPCHK(mesh::launch_select_count(mode, v.flags, v.N, L->counts, total, v.stream));
+    HIPCHK(hipMemcpyAsync(&L->n, total, 4, hipMemcpyDeviceToHost, v.stream));
     HIPCHK(hipStreamSynchronize(v.stream));
     const size_t n = L->n ? L->n : 1;
-    HIPCHK(hipMalloc((void**)&L->pos, n * sizeof(float4)));
-    HIPCHK(hipMalloc((void**)&L->val, n * sizeof(float4)));
-    mesh::Sources s{L->pos, L->val, L->total};
-    HIPCHK(mesh::launch_select_scatter(mode, v.flags, v.b_dyn, v.N, v.nx, v.ny, L->counts, s, v.stream));
+    const bool group = mesh::shifts_possible(L->n, v.N);
+    HIPCHK(hipMalloc((void**)&L->data, n * (group ? 3 * sizeof(float4) + 2 * sizeof(int2) + 2 * sizeof(uint32_t) : 2 * sizeof(float4)) + 4));
+    float4* const d = (float4*)L->data;
+    L->src = mesh::Sources{d, d + n, total};
+    HIPCHK(mesh::launch_select_scatter(mode, v.flags, v.b_dyn, v.N, v.nx, v.ny, L->counts, L->src, v.stream));
+    if (!group) return ION_OK;
+    int2* const c = (int2*)(d + 3 * n);
+    uint32_t* const g = (uint32_t*)(c + 2 * n);
+    uint32_t found[2];
+    L->shifts = mesh::ShiftLists{g, d + 2 * n, c, c + n, g + n, total + 2, 0, 0};
+    HIPCHK(mesh::launch_group(mode, L->src, L->shifts, v.stream));
+    HIPCHK(hipMemcpyAsync(found, total + 2, 8, hipMemcpyDeviceToHost, v.stream));
+    HIPCHK(hipStreamSynchronize(v.stream));
+    L->shifts.ngroup = found[0];
+    L->shifts.nbatch = found[1];
     return ION_OK;
 }
 
@@ -352,8 +362,7 @@ int ion_precompute_b(ion_handle* h) {
         HIPCHK(hipMalloc((void**)&tmp, Np * sizeof(float)));
         psi = tmp;
     }
-    mesh::Sources s{L.pos, L.val, L.total};
-    hipError_t e = mesh::launch_psi(s, psi, v.nx, v.ny, v.nz, v.stream);
+    hipError_t e = mesh::launch_psi(L.src, L.n, L.shifts, psi, v.nx, v.ny, v.nz, v.stream);
     if (e == hipSuccess) e = mesh::launch_static_b(v.flags, v.b_stat, psi, v.nx, v.ny, v.nz, v.kc->kmu0, v.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
     (void)hipFree(tmp);
@@ -374,8 +383,7 @@ int ion_precompute_e_ecr(ion_handle* h) {
     if (!v.e_var) return fail(ION_ERR_INVALID, "precompute_E_ECR needs ext_magneto_hydro and ext_subgrid_ecr");
     SourceList L;
     if ((rc = select_sources(v, 1, &L))) return rc;
-    mesh::Sources s{L.pos, L.val, L.total};
-    hipError_t e = mesh::launch_static_e(s, v.flags, v.e_var, v.nx, v.ny, v.nz, v.kc->ke, v.stream);
+    hipError_t e = mesh::launch_static_e(L.src, L.n, L.shifts, v.flags, v.e_var, v.nx, v.ny, v.nz, v.kc->ke, v.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
     if (e != hipSuccess) return fail(ION_ERR_DEVICE, std::string("precompute_E_ECR: ") + hipGetErrorString(e));
     return ION_OK;
@@ -387,8 +395,7 @@ int ion_precompute_e(ion_handle* h) {
     if (rc || (rc = need_mhd(v, "precompute_E"))) return rc;
     SourceList L;
     if ((rc = select_sources(v, 1, &L))) return rc;
-    mesh::Sources s{L.pos, L.val, L.total};
-    hipError_t e = mesh::launch_static_e(s, v.flags, v.e_stat, v.nx, v.ny, v.nz, v.kc->ke, v.stream);
+    hipError_t e = mesh::launch_static_e(L.src, L.n, L.shifts, v.flags, v.e_stat, v.nx, v.ny, v.nz, v.kc->ke, v.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
     if (e != hipSuccess) return fail(ION_ERR_DEVICE, std::string("precompute_E: ") + hipGetErrorString(e));
     return ION_OK;
