@@ -11,6 +11,17 @@ enum StoreKind { STORE_FP16S = 0, STORE_FP16C = 1, STORE_FP32 = 2, STORE_FP64 = 
 // Arguments of initialize / stream_collide / update_fields. Buffers are the
 // reference's device buffers (src/lbm/domain.rs:151-211), all SoA:
 // scalar fields [N], vector fields [3][N], DDFs [q][N].
+// Division of n < 2^30 by d >= 1: (4 n m) >> 32 >> s with s = ceil(log2 d),
+// m = floor(2^(30 + s) / d) + 1, whose error d m - 2^(30 + s) is at most 2^s.
+struct FastDiv {
+    uint32_t m, s;
+};
+inline FastDiv fast_div(uint32_t d) {
+    uint32_t s = 0;
+    while (s < 31u && (1u << s) < d) s++;
+    return FastDiv{(uint32_t)(((uint64_t)1 << (30 + s)) / d + 1u), s};
+}
+
 struct LbmArgs {
     void* fi;
     float* rho;
@@ -26,7 +37,9 @@ struct LbmArgs {
     float* q;             // cell charge
     float4* lod_seg;      // level-1 LOD row-segment sums [N / lod_bx]
     uint32_t nx, ny, nz;
-    uint32_t pad0;
+    float lim;            // 16-bit storage: bound of density, force and speed sums below which a stored value
+                          // is finite and below 2^112 (0: none)
+    FastDiv div_x, div_xy;  // by nx and nx ny
     uint64_t N;
     uint64_t N_store;     // == N; a separate argument so that the compiler computes the
                           // store-side slot bases at the stores instead of keeping the

@@ -17,23 +17,29 @@ struct Nbr {
     uint32_t x0, xp, xm, y0, yp, ym, z0, zp, zm;
 };
 
+__device__ __forceinline__ uint32_t fdiv(uint32_t n, FastDiv d) { return __umulhi(n << 2, d.m) >> d.s; }
+
+// How a kernel reaches the DDFs. MEM_ROWS: every wavefront lies in one row (NX
+// a multiple of 64), so the offsets of y and z are scalars. MEM_CACHED: plain
+// accesses instead of nontemporal ones.
+enum { MEM_CELLS = 0, MEM_ROWS = 1, MEM_CACHED = 2 };
+
 // calculate_indices, sim_kernels.cl:248-259 (periodic wrap)
-__device__ __forceinline__ Nbr neighbours(uint32_t n, uint32_t NX, uint32_t NY, uint32_t NZ) {
-    const uint32_t nxy = NX * NY;
-    const uint32_t z = n / nxy;
-    const uint32_t t = n - z * nxy;
-    const uint32_t y = t / NX;
-    const uint32_t x = t - y * NX;
+template <int MEM = MEM_CELLS> __device__ __forceinline__ Nbr neighbours(uint32_t n, const LbmArgs& a) {
+    const uint32_t NX = a.nx, nxy = NX * a.ny;
+    const uint32_t m = MEM == MEM_ROWS ? (uint32_t)__builtin_amdgcn_readfirstlane((int)n) : n;
+    const uint32_t row = fdiv(m, a.div_x) * NX;  // first cell of the row
+    const uint32_t x = n - row;
     Nbr b;
     b.x0 = x;
     b.xp = (x + 1u == NX) ? 0u : x + 1u;
     b.xm = (x == 0u) ? NX - 1u : x - 1u;
-    b.y0 = y * NX;
-    b.yp = ((y + 1u == NY) ? 0u : y + 1u) * NX;
-    b.ym = ((y == 0u) ? NY - 1u : y - 1u) * NX;
-    b.z0 = z * nxy;
-    b.zp = ((z + 1u == NZ) ? 0u : z + 1u) * nxy;
-    b.zm = ((z == 0u) ? NZ - 1u : z - 1u) * nxy;
+    b.z0 = fdiv(m, a.div_xy) * nxy;
+    b.zp = (b.z0 + nxy == (uint32_t)a.N) ? 0u : b.z0 + nxy;
+    b.zm = (b.z0 == 0u ? (uint32_t)a.N : b.z0) - nxy;
+    b.y0 = row - b.z0;
+    b.yp = (b.y0 + NX == nxy) ? 0u : b.y0 + NX;
+    b.ym = (b.y0 == 0u ? nxy : b.y0) - NX;
     return b;
 }
 
@@ -72,6 +78,28 @@ template <class T> __device__ __forceinline__ const T* at(const T* base, uint32_
     return (const T*)((const char*)base + (uint32_t)(idx * (uint32_t)sizeof(T)));
 }
 
+// Element of the cell at neighbour offsets (cx, cy, cz) of `base`: by the row's
+// scalar offset and the cell's along x, or by the index.
+template <int MEM, int CX, int CY, int CZ, class T> __device__ __forceinline__ T* nb_at(T* base, const Nbr& b) {
+    const uint32_t x = CX == 0 ? b.x0 : (CX > 0 ? b.xp : b.xm);
+    const uint32_t y = CY == 0 ? b.y0 : (CY > 0 ? b.yp : b.ym);
+    const uint32_t z = CZ == 0 ? b.z0 : (CZ > 0 ? b.zp : b.zm);
+    if constexpr (MEM == MEM_ROWS) return at(base + (y + z), x);
+    else return at(base, x + y + z);
+}
+template <int MEM, int Q, int I, class T> __device__ __forceinline__ T* nb_at(T* base, const Nbr& b) {
+    return nb_at<MEM, VS<Q>::cx[I], VS<Q>::cy[I], VS<Q>::cz[I]>(base, b);
+}
+
+template <int MEM, class T> __device__ __forceinline__ T ddf_ld(const T* p) {
+    if constexpr (MEM == MEM_CACHED) return *p;
+    else return __builtin_nontemporal_load(p);
+}
+template <int MEM, class T> __device__ __forceinline__ void ddf_st(T v, T* p) {
+    if constexpr (MEM == MEM_CACHED) *p = v;
+    else __builtin_nontemporal_store(v, p);
+}
+
 // Esoteric-pull load/store of an NQ-direction lattice (load_f/store_f and
 // load_a/store_a, sim_kernels.cl:234-247, 397-410). Direction pair (i, i+1)
 // of cell n lives in slots (n, i+1) and (j[i], i) on even steps and in
@@ -93,17 +121,16 @@ __device__ __forceinline__ void load_ddfs(const typename S::T* __restrict__ buf,
 }
 // Raw (undecoded) esoteric-pull loads, so that a kernel can issue the loads
 // of all its lattices before the first decode and keep them in flight together.
-template <int Q, int NQ, class S>
+template <int MEM, int Q, int NQ, class S>
 __device__ __forceinline__ void load_raw(const typename S::T* __restrict__ buf, uint64_t N, uint32_t n, const Nbr& b,
                                          uint32_t odd, typename S::T* raw) {
     raw[0] = *at(buf, n);
     static_for<(NQ - 1) / 2>([&](auto p) {
         constexpr int i = 2 * decltype(p)::value + 1;
-        const uint32_t j = nb_index<Q, i>(b);
         const typename S::T* so = buf + (uint64_t)(i + 1u - odd) * N;
         const typename S::T* sn = buf + (uint64_t)(i + odd) * N;
-        raw[i] = __builtin_nontemporal_load(at(so, n));
-        raw[i + 1] = __builtin_nontemporal_load(at(sn, j));
+        raw[i] = ddf_ld<MEM>(at(so, n));
+        raw[i + 1] = ddf_ld<MEM>(nb_at<MEM, Q, i>(sn, b));
     });
 }
 template <int NQ, class S>
@@ -112,17 +139,16 @@ __device__ __forceinline__ void decode(const typename S::T* raw, typename S::R* 
     for (int i = 0; i < NQ; i++) fh[i] = S::ld(raw[i]);
 }
 
-template <int Q, int NQ, class S>
+template <int MEM, int Q, int NQ, class S>
 __device__ __forceinline__ void store_ddfs(typename S::T* __restrict__ buf, uint64_t N, uint32_t n, const Nbr& b,
                                            uint32_t odd, const typename S::R* fh) {
     *at(buf, n) = S::st(fh[0]);
     static_for<(NQ - 1) / 2>([&](auto p) {
         constexpr int i = 2 * decltype(p)::value + 1;
-        const uint32_t j = nb_index<Q, i>(b);
         typename S::T* so = buf + (uint64_t)(i + 1u - odd) * N;
         typename S::T* sn = buf + (uint64_t)(i + odd) * N;
-        __builtin_nontemporal_store(S::st(fh[i]), at(sn, j));
-        __builtin_nontemporal_store(S::st(fh[i + 1]), at(so, n));
+        ddf_st<MEM>(S::st(fh[i]), nb_at<MEM, Q, i>(sn, b));
+        ddf_st<MEM>(S::st(fh[i + 1]), at(so, n));
     });
 }
 
@@ -153,40 +179,36 @@ template <int Q, int NQ> __device__ __forceinline__ constexpr int xslots() {
 }
 // store_ddfs with the +x neighbour stores deposited in xch[(XB + slot) * W + dst]
 // (dst: the target cell's work-item in the block, XCH_NONE: store directly)
-template <int Q, int NQ, class S, int XB>
+template <int MEM, int Q, int NQ, class S, int XB>
 __device__ __forceinline__ void store_ddfs_x(typename S::T* __restrict__ buf, uint64_t N, uint32_t n, const Nbr& b,
                                              uint32_t odd, const typename S::R* fh, typename S::T* xch, uint32_t W,
                                              uint32_t dst) {
     *at(buf, n) = S::st(fh[0]);
     static_for<(NQ - 1) / 2>([&](auto p) {
         constexpr int i = 2 * decltype(p)::value + 1;
-        const uint32_t j = nb_index<Q, i>(b);
         typename S::T* so = buf + (uint64_t)(i + 1u - odd) * N;
         typename S::T* sn = buf + (uint64_t)(i + odd) * N;
         constexpr int ks = xslot<Q, i>();
         if constexpr (ks >= 0) {
             if (dst != XCH_NONE) xch[(uint32_t)(XB + ks) * W + dst] = S::st(fh[i]);
-            else __builtin_nontemporal_store(S::st(fh[i]), at(sn, j));
+            else ddf_st<MEM>(S::st(fh[i]), nb_at<MEM, Q, i>(sn, b));
         } else {
-            __builtin_nontemporal_store(S::st(fh[i]), at(sn, j));
+            ddf_st<MEM>(S::st(fh[i]), nb_at<MEM, Q, i>(sn, b));
         }
-        __builtin_nontemporal_store(S::st(fh[i + 1]), at(so, n));
+        ddf_st<MEM>(S::st(fh[i + 1]), at(so, n));
     });
 }
 // the stores handed to this cell: slot (i + odd, n + c_i - x) of every +x direction i,
 // i.e. the neighbour index of the source cell, one cell back along x
-template <int Q, int NQ, class S, int XB>
+template <int MEM, int Q, int NQ, class S, int XB>
 __device__ __forceinline__ void store_received(typename S::T* __restrict__ buf, uint64_t N, const Nbr& b,
                                                uint32_t odd, const typename S::T* xch, uint32_t W, uint32_t tid) {
     static_for<(NQ - 1) / 2>([&](auto p) {
         constexpr int i = 2 * decltype(p)::value + 1;
         constexpr int ks = xslot<Q, i>();
         if constexpr (ks >= 0) {
-            constexpr int cy = VS<Q>::cy[i], cz = VS<Q>::cz[i];
-            const uint32_t y = cy == 0 ? b.y0 : (cy > 0 ? b.yp : b.ym);
-            const uint32_t z = cz == 0 ? b.z0 : (cz > 0 ? b.zp : b.zm);
             typename S::T* sn = buf + (uint64_t)(i + odd) * N;
-            __builtin_nontemporal_store(xch[(uint32_t)(XB + ks) * W + tid], at(sn, b.x0 + y + z));
+            ddf_st<MEM>(xch[(uint32_t)(XB + ks) * W + tid], (nb_at<MEM, 0, VS<Q>::cy[i], VS<Q>::cz[i]>(sn, b)));
         }
     });
 }
@@ -196,22 +218,21 @@ __device__ __forceinline__ void store_received(typename S::T* __restrict__ buf, 
 // once all three lattices are done), and the stores of captured codes
 // (store_cap: the cell's own targets; store_received_codes: the targets of the
 // cell one back along x, one cell back from this cell's neighbours)
-template <int Q, int NQ, class S>
+template <int MEM, int Q, int NQ, class S>
 __device__ __forceinline__ void store_ddfs_cap(typename S::T* __restrict__ buf, uint64_t N, uint32_t n, const Nbr& b,
                                                uint32_t odd, const typename S::R* fh, typename S::T* cap) {
     *at(buf, n) = S::st(fh[0]);
     static_for<(NQ - 1) / 2>([&](auto p) {
         constexpr int i = 2 * decltype(p)::value + 1;
-        const uint32_t j = nb_index<Q, i>(b);
         typename S::T* so = buf + (uint64_t)(i + 1u - odd) * N;
         typename S::T* sn = buf + (uint64_t)(i + odd) * N;
         constexpr int ks = xslot<Q, i>();
         if constexpr (ks >= 0) cap[ks] = S::st(fh[i]);
-        else __builtin_nontemporal_store(S::st(fh[i]), at(sn, j));
-        __builtin_nontemporal_store(S::st(fh[i + 1]), at(so, n));
+        else ddf_st<MEM>(S::st(fh[i]), nb_at<MEM, Q, i>(sn, b));
+        ddf_st<MEM>(S::st(fh[i + 1]), at(so, n));
     });
 }
-template <int Q, int NQ, class S>
+template <int MEM, int Q, int NQ, class S>
 __device__ __forceinline__ void store_cap(typename S::T* __restrict__ buf, uint64_t N, const Nbr& b, uint32_t odd,
                                           const typename S::T* cap) {
     static_for<(NQ - 1) / 2>([&](auto p) {
@@ -219,22 +240,19 @@ __device__ __forceinline__ void store_cap(typename S::T* __restrict__ buf, uint6
         constexpr int ks = xslot<Q, i>();
         if constexpr (ks >= 0) {
             typename S::T* sn = buf + (uint64_t)(i + odd) * N;
-            __builtin_nontemporal_store(cap[ks], at(sn, nb_index<Q, i>(b)));
+            ddf_st<MEM>(cap[ks], nb_at<MEM, Q, i>(sn, b));
         }
     });
 }
-template <int Q, int NQ, class S>
+template <int MEM, int Q, int NQ, class S>
 __device__ __forceinline__ void store_received_codes(typename S::T* __restrict__ buf, uint64_t N, const Nbr& b,
                                                      uint32_t odd, const typename S::T* code) {
     static_for<(NQ - 1) / 2>([&](auto p) {
         constexpr int i = 2 * decltype(p)::value + 1;
         constexpr int ks = xslot<Q, i>();
         if constexpr (ks >= 0) {
-            constexpr int cy = VS<Q>::cy[i], cz = VS<Q>::cz[i];
-            const uint32_t y = cy == 0 ? b.y0 : (cy > 0 ? b.yp : b.ym);
-            const uint32_t z = cz == 0 ? b.z0 : (cz > 0 ? b.zp : b.zm);
             typename S::T* sn = buf + (uint64_t)(i + odd) * N;
-            __builtin_nontemporal_store(code[ks], at(sn, b.x0 + y + z));
+            ddf_st<MEM>(code[ks], (nb_at<MEM, 0, VS<Q>::cy[i], VS<Q>::cz[i]>(sn, b)));
         }
     });
 }
@@ -264,7 +282,7 @@ __global__ void __launch_bounds__(256) k_initialize(LbmArgs a) {
     if (n64 >= a.N) return;
     const uint32_t n = (uint32_t)n64;
     const uint64_t N = a.N;
-    const Nbr b = neighbours(n, a.nx, a.ny, a.nz);
+    const Nbr b = neighbours(n, a);
     const uint8_t bo = a.flags[n] & 0x1F;
     if (bo == 0x01) {
         U[n] = R(0);
@@ -275,11 +293,11 @@ __global__ void __launch_bounds__(256) k_initialize(LbmArgs a) {
     const R ux = U[n], uy = U[N + n], uz = U[2 * N + n];
     R fe[Q];
     f_eq<Q>(Rho[n], ux, uy, uz, fe);
-    store_ddfs<Q, Q, S>((typename S::T*)a.fi, N, n, b, 1u, fe);
+    store_ddfs<MEM_CELLS, Q, Q, S>((typename S::T*)a.fi, N, n, b, 1u, fe);
     if (MHD) {
         R qeq[7];
         a_eq(Qp[n], ux, uy, uz, qeq);
-        store_ddfs<19, 7, S>((typename S::T*)a.fqi, N, n, b, 1u, qeq);
+        store_ddfs<MEM_CELLS, 19, 7, S>((typename S::T*)a.fqi, N, n, b, 1u, qeq);
 #pragma unroll
         for (int k = 0; k < 3; k++) {
             Bd[k * N + n] = Bs[k * N + n];
@@ -288,10 +306,10 @@ __global__ void __launch_bounds__(256) k_initialize(LbmArgs a) {
         // sim_kernels.cl:823-825 writes density 0; a non-zero ei_rho0 (build
         // extension) starts the electron gas of non-solid cells at that density
         f_eq<Q>(bo == 0x01 ? R(0) : R(a.ei_rho0), ux, uy, uz, fe);
-        store_ddfs<Q, Q, S>((typename S::T*)a.ei, N, n, b, 1u, fe);
+        store_ddfs<MEM_CELLS, Q, Q, S>((typename S::T*)a.ei, N, n, b, 1u, fe);
         if constexpr (ECR) {  // electron temperature DDFs, sim_kernels.cl:827-831
             a_eq(R(a.et[n]), ux, uy, uz, qeq);
-            store_ddfs<19, 7, S>((typename S::T*)a.eti, N, n, b, 1u, qeq);
+            store_ddfs<MEM_CELLS, 19, 7, S>((typename S::T*)a.eti, N, n, b, 1u, qeq);
         }
     }
 }
@@ -303,12 +321,17 @@ __global__ void __launch_bounds__(256) k_initialize(LbmArgs a) {
 // summed per segment by the pairwise tree in LDS and written to lod_seg.
 // ---------------------------------------------------------------------------
 // MHD variants with 32-bit arithmetic are held to 128 VGPRs (4 wavefronts per
-// SIMD); with the neighbour offsets recomputed before the stores they need
-// 111-114, and holding them to 96 (5 wavefronts) spills 14-20.
-template <int Q, class S, bool MHD, bool TRT, bool LOD, bool ECR = false>
+// SIMD); holding them to 96 (5 wavefronts) spills.
+// Bound by memory. us a step, with divisions for the cell's coordinates, vector
+// offsets of every neighbour, ten operations an encoded and five a decoded
+// 16-bit value / now: D3Q19 FP16C 256^3 358 / 334 (658 / 458 vector operations
+// a wavefront), MHD FP16C 256^3 876 / 860 (1896 / 1516), MHD FP32 256^3 1257 /
+// 1243. Small lattices: the rule at the launch (CACHED_BYTES).
+template <int Q, class S, bool MHD, bool TRT, bool LOD, bool ECR = false, int MEM = MEM_CELLS>
 __global__ void __launch_bounds__(MHD ? 512 : 256)
     __attribute__((amdgpu_waves_per_eu(MHD && !ECR && sizeof(typename S::R) == 4 ? 4 : 1))) k_stream_collide(LbmArgs a) {
     typedef typename S::R R;
+    typedef std::conditional_t<ECR, S, Finite<S>> FS;  // stores: values are checked first (tame)
     typedef typename V4<R>::T V4;
     (void)sizeof(V4);
     R* const Rho = (R*)a.rho;
@@ -332,8 +355,6 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
     const uint32_t n = (uint32_t)n64;
     bool active = n64 < N;
     uint8_t bo = 0x01;
-    if (active) bo = *at(a.flags, n) & 0x1F;
-    active = active && bo != 0x01;
     V4 lod = mk4<R>(R(0), R(0), R(0), R(0));
     typedef typename S::T T;
     // +x neighbour stores through LDS: the D3Q19 MHD variants with the fused LOD
@@ -365,30 +386,77 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
     };
     (void)xdst;
 
+    // every load of the cell first: fi, ei, fqi, E_dyn, B_dyn; where the
+    // latency counts, before its flag is known
+    T rf[Q], re[MHD ? Q : 1], rq[MHD ? 7 : 1], rt[ECR ? 7 : 1];
+    R Bx = R(0), By = R(0), Bz = R(0), Ex = R(0), Ey = R(0), Ez = R(0);
+    auto load = [&](const Nbr& b) {
+        load_raw<MEM, Q, Q, S>((const T*)a.fi, N, n, b, a.odd, rf);
+        if constexpr (MHD) {
+            load_raw<MEM, Q, Q, S>((const T*)a.ei, N, n, b, a.odd, re);
+            load_raw<MEM, 19, 7, S>((const T*)a.fqi, N, n, b, a.odd, rq);
+            if constexpr (ECR) load_raw<MEM, 19, 7, S>((const T*)a.eti, N, n, b, a.odd, rt);
+            Bx = *at(Bd, n); By = *at(Bd + N, n); Bz = *at(Bd + 2 * N, n);
+            Ex = *at(Ed, n); Ey = *at(Ed + N, n); Ez = *at(Ed + 2 * N, n);
+        }
+    };
+    Nbr b;
+    if constexpr (MEM == MEM_CACHED) {
+        if (n64 < N) {
+            b = neighbours<MEM>(n, a);
+            load(b);
+        }
+    }
+    if (active) bo = *at(a.flags, n) & 0x1F;
+    active = active && bo != 0x01;
     if (active) {
         const bool is_e = a.eqb && bo == 0x02;
-        const Nbr b = neighbours(n, a.nx, a.ny, a.nz);
+        if constexpr (MEM != MEM_CACHED) b = neighbours<MEM>(n, a);
         // MHD: the neighbour offsets again before each store instead of nine
         // registers held from the loads to the last store (the 32-bit MHD
         // variants are at their 128-register limit); the empty asm keeps the
         // compiler from reusing b
         auto nb_store = [&]() -> Nbr {
-            if constexpr (!MHD) return b;
+            if constexpr (!MHD || MEM == MEM_ROWS) return b;
             uint32_t m = n;
             __asm__ volatile("" : "+v"(m));
-            return neighbours(m, a.nx, a.ny, a.nz);
+            return neighbours(m, a);
         };
-        // every load of the cell first: fi, ei, fqi, E_dyn, B_dyn
-        T rf[Q], re[MHD ? Q : 1], rq[MHD ? 7 : 1], rt[ECR ? 7 : 1];
-        R Bx = R(0), By = R(0), Bz = R(0), Ex = R(0), Ey = R(0), Ez = R(0);
-        load_raw<Q, Q, S>((const T*)a.fi, N, n, b, a.odd, rf);
-        if (MHD) {
-            load_raw<Q, Q, S>((const T*)a.ei, N, n, b, a.odd, re);
-            load_raw<19, 7, S>((const T*)a.fqi, N, n, b, a.odd, rq);
-            if constexpr (ECR) load_raw<19, 7, S>((const T*)a.eti, N, n, b, a.odd, rt);
-            Bx = *at(Bd, n); By = *at(Bd + N, n); Bz = *at(Bd + 2 * N, n);
-            Ex = *at(Ed, n); Ey = *at(Ed + N, n); Ez = *at(Ed + 2 * N, n);
-        }
+        // Stored values are finite and below 2^112 if s < lim. If a wavefront
+        // has a cell where it is not (wild), they are replaced by what their
+        // general code decodes to, which has the same code (tame).
+        auto fabsR = [](R x) -> R {
+            if constexpr (sizeof(R) == 4) return __builtin_fabsf(x);
+            else return __builtin_fabs(x);
+        };
+        auto wild = [&](R p, R x, R y, R z) -> bool {
+            if constexpr (!ECR && sizeof(T) == 2)
+                return __ballot(!(fabsR(p) + fabsR(x) + fabsR(y) + fabsR(z) < R(a.lim))) != 0ull;
+            else return false;
+        };
+        auto tame = [&](bool any, R* f, auto num) {
+            if constexpr (!ECR && sizeof(T) == 2) {
+                if (__builtin_expect(any, 0)) {
+#pragma unroll
+                    for (int i = 0; i < decltype(num)::value; i++) f[i] = S::ld(S::st(f[i]));
+                }
+            }
+        };
+        // TYPE_E cells take the equilibrium: without the selections where a
+        // wavefront has none (MHD; the fluid kernels keep more wavefronts in
+        // flight with the equilibrium's values used as they are computed)
+        constexpr bool SPLIT = MHD && !ECR && sizeof(R) == 4;
+        const bool any_e = !SPLIT || __ballot(is_e) != 0ull;
+        auto relax = [&](R* f, const R* eq, auto&& val) {
+            if (!any_e) {
+#pragma unroll
+                for (int i = 0; i < Q; i++) f[i] = val(i);
+            } else {
+#pragma unroll
+                for (int i = 0; i < Q; i++) f[i] = is_e ? eq[i] : val(i);
+            }
+        };
+        if constexpr (MEM != MEM_CACHED) load(b);
         R fhn[Q];
         decode<Q, S>(rf, fhn);
         R rhon, uxn, uyn, uzn;
@@ -462,7 +530,7 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
                 const R wq = WQ;
 #pragma unroll
                 for (int i = 0; i < 7; i++) ethn[i] = fmaR(R(1) - wq, ethn[i], wq * eteq[i]);
-                store_ddfs<19, 7, S>((T*)a.eti, a.N_store, n, b, a.odd, ethn);
+                store_ddfs<MEM, 19, 7, S>((T*)a.eti, a.N_store, n, b, a.odd, ethn);
                 const R dq = R(0.0001f) * Etn;  // ionisation
                 rhon_e += dq;
                 rhon_q += dq;
@@ -478,9 +546,10 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
             const R wq = WQ;
 #pragma unroll
             for (int i = 0; i < 7; i++) qhn[i] = inlet ? qeq[i] : fmaR(R(1) - wq, qhn[i], wq * qeq[i]);
-            if constexpr (XCH) store_ddfs_x<19, 7, S, 2 * xslots<19, 19>()>((T*)a.fqi, a.N_store, n, nb_store(), a.odd, qhn, xch, BW, xdst(b.x0));
-            else if constexpr (XCH16) store_ddfs_cap<19, 7, S>((T*)a.fqi, a.N_store, n, nb_store(), a.odd, qhn, cap_q);
-            else store_ddfs<19, 7, S>((T*)a.fqi, a.N_store, n, nb_store(), a.odd, qhn);
+            tame(wild(rhon_q, uxn, uyn, uzn), qhn, std::integral_constant<int, 7>{});
+            if constexpr (XCH) store_ddfs_x<MEM, 19, 7, FS, 2 * xslots<19, 19>()>((T*)a.fqi, a.N_store, n, nb_store(), a.odd, qhn, xch, BW, xdst(b.x0));
+            else if constexpr (XCH16) store_ddfs_cap<MEM, 19, 7, FS>((T*)a.fqi, a.N_store, n, nb_store(), a.odd, qhn, cap_q);
+            else store_ddfs<MEM, 19, 7, FS>((T*)a.fqi, a.N_store, n, nb_store(), a.odd, qhn);
             // electron gas part 2: F = -rho_e (E + u_e x B), Guo forcing, SRT
             const R crx = uyn_e * Bz - uzn_e * By;
             const R cry = uzn_e * Bx - uxn_e * Bz;
@@ -490,16 +559,14 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
             uxn_e = clampR(fmaR(efx, rho2_e, uxn_e), -C, C);
             uyn_e = clampR(fmaR(efy, rho2_e, uyn_e), -C, C);
             uzn_e = clampR(fmaR(efz, rho2_e, uzn_e), -C, C);
+            const bool wild_e = wild(rhon_e, efx, efy, efz);
             forcing<Q>(uxn_e, uyn_e, uzn_e, efx, efy, efz, Fin);
             f_eq<Q>(rhon_e, uxn_e, uyn_e, uzn_e, feq);
-#pragma unroll
-            for (int i = 0; i < Q; i++) {
-                const R fi = Fin[i] * c_tau;
-                ehn[i] = is_e ? feq[i] : fmaR(R(1) - w, ehn[i], fmaR(w, feq[i], fi));
-            }
-            if constexpr (XCH) store_ddfs_x<Q, Q, S, xslots<19, 19>()>((T*)a.ei, a.N_store, n, nb_store(), a.odd, ehn, xch, BW, xdst(b.x0));
-            else if constexpr (XCH16) store_ddfs_cap<Q, Q, S>((T*)a.ei, a.N_store, n, nb_store(), a.odd, ehn, cap_e);
-            else store_ddfs<Q, Q, S>((T*)a.ei, a.N_store, n, nb_store(), a.odd, ehn);
+            relax(ehn, feq, [&](int i) { return fmaR(R(1) - w, ehn[i], fmaR(w, feq[i], Fin[i] * c_tau)); });
+            tame(wild_e, ehn, std::integral_constant<int, Q>{});
+            if constexpr (XCH) store_ddfs_x<MEM, Q, Q, FS, xslots<19, 19>()>((T*)a.ei, a.N_store, n, nb_store(), a.odd, ehn, xch, BW, xdst(b.x0));
+            else if constexpr (XCH16) store_ddfs_cap<MEM, Q, Q, FS>((T*)a.ei, a.N_store, n, nb_store(), a.odd, ehn, cap_e);
+            else store_ddfs<MEM, Q, Q, FS>((T*)a.ei, a.N_store, n, nb_store(), a.odd, ehn);
             // EM force on the gas (plain multiply-add, as written)
             fxn += rhon_q * (Ex + uyn * Bz - uzn * By);
             fyn += rhon_q * (Ey + uzn * Bx - uxn * Bz);
@@ -511,7 +578,7 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
             uxn = clampR(fmaR(fxn, rho2, uxn), -C, C);
             uyn = clampR(fmaR(fyn, rho2, uyn), -C, C);
             uzn = clampR(fmaR(fzn, rho2, uzn), -C, C);
-            forcing<Q>(uxn, uyn, uzn, fxn, fyn, fzn, Fin);
+            if constexpr (TRT || !SPLIT) forcing<Q>(uxn, uyn, uzn, fxn, fyn, fzn, Fin);
         } else {
             uxn = clampR(uxn, -C, C);
             uyn = clampR(uyn, -C, C);
@@ -525,13 +592,19 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
             *at(U + N, n) = uyn;
             *at(U + 2 * N, n) = uzn;
         }
+        const bool wild_f = wild(rhon, fxn, fyn, fzn);
         f_eq<Q>(rhon, uxn, uyn, uzn, feq);
         if (!TRT) {
-            const bool vf = a.vforce != 0;
-#pragma unroll
-            for (int i = 0; i < Q; i++) {
-                const R fi = vf ? Fin[i] * c_tau : Fin[i];
-                fhn[i] = is_e ? feq[i] : fmaR(R(1) - w, fhn[i], fmaR(w, feq[i], fi));
+            if constexpr (SPLIT) {
+                if (a.vforce) {
+                    forcing<Q>(uxn, uyn, uzn, fxn, fyn, fzn, Fin);
+                    relax(fhn, feq, [&](int i) { return fmaR(R(1) - w, fhn[i], fmaR(w, feq[i], Fin[i] * c_tau)); });
+                } else {
+                    relax(fhn, feq, [&](int i) { return fmaR(R(1) - w, fhn[i], fmaR(w, feq[i], R(0))); });
+                }
+            } else {
+                const bool vf = a.vforce != 0;
+                relax(fhn, feq, [&](int i) { return fmaR(R(1) - w, fhn[i], fmaR(w, feq[i], vf ? Fin[i] * c_tau : Fin[i])); });
             }
         } else {
             const R wp = w;
@@ -558,15 +631,15 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
                 feb[i] = feq[i + 1];
                 feb[i + 1] = feq[i];
             }
-#pragma unroll
-            for (int i = 0; i < Q; i++)
-                fhn[i] = is_e ? feq[i]
-                              : fmaR(R(0.5) * wp, feq[i] - fhn[i] + feb[i] - fhb[i],
-                                               fmaR(R(0.5) * wm, feq[i] - feb[i] - fhn[i] + fhb[i], fhn[i] + Fin[i]));
+            relax(fhn, feq, [&](int i) {
+                return fmaR(R(0.5) * wp, feq[i] - fhn[i] + feb[i] - fhb[i],
+                            fmaR(R(0.5) * wm, feq[i] - feb[i] - fhn[i] + fhb[i], fhn[i] + Fin[i]));
+            });
         }
-        if constexpr (XCH) store_ddfs_x<Q, Q, S, 0>((T*)a.fi, a.N_store, n, nb_store(), a.odd, fhn, xch, BW, xdst(b.x0));
+        tame(wild_f, fhn, std::integral_constant<int, Q>{});
+        if constexpr (XCH) store_ddfs_x<MEM, Q, Q, FS, 0>((T*)a.fi, a.N_store, n, nb_store(), a.odd, fhn, xch, BW, xdst(b.x0));
         else if constexpr (XCH16) {
-            store_ddfs_cap<Q, Q, S>((T*)a.fi, a.N_store, n, nb_store(), a.odd, fhn, cap_f);
+            store_ddfs_cap<MEM, Q, Q, FS>((T*)a.fi, a.N_store, n, nb_store(), a.odd, fhn, cap_f);
             const uint32_t dst = xdst(b.x0);
             if (dst != XCH_NONE) {  // to the work-item of cell n + 1 along x, two codes per word
                 auto pk = [](uint16_t lo, uint16_t hi) { return (uint32_t)lo | ((uint32_t)hi << 16); };
@@ -578,12 +651,12 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
                 xch32[5 * BW + dst] = (uint32_t)cap_q[0];
             } else {  // the target leaves the block: store directly
                 const Nbr bs = nb_store();
-                store_cap<Q, Q, S>((T*)a.fi, a.N_store, bs, a.odd, cap_f);
-                store_cap<Q, Q, S>((T*)a.ei, a.N_store, bs, a.odd, cap_e);
-                store_cap<19, 7, S>((T*)a.fqi, a.N_store, bs, a.odd, cap_q);
+                store_cap<MEM, Q, Q, S>((T*)a.fi, a.N_store, bs, a.odd, cap_f);
+                store_cap<MEM, Q, Q, S>((T*)a.ei, a.N_store, bs, a.odd, cap_e);
+                store_cap<MEM, 19, 7, S>((T*)a.fqi, a.N_store, bs, a.odd, cap_q);
             }
         }
-        else store_ddfs<Q, Q, S>((T*)a.fi, a.N_store, n, nb_store(), a.odd, fhn);
+        else store_ddfs<MEM, Q, Q, FS>((T*)a.fi, a.N_store, n, nb_store(), a.odd, fhn);
     }
 
     if (LOD) {
@@ -594,7 +667,7 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
         __syncthreads();
         if constexpr (XCH16) {
             if (n64 < N) {
-                const Nbr br = neighbours(n, a.nx, a.ny, a.nz);
+                const Nbr br = neighbours<MEM>(n, a);
                 const uint32_t NX = a.nx;
                 const uint32_t src = NX <= BW ? (br.x0 == 0u ? tid + NX - 1u : tid - 1u) : (tid > 0u ? tid - 1u : XCH_NONE);
                 if (src != XCH_NONE && xfl[src]) {
@@ -604,9 +677,9 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
                     const T rf[5] = {(T)w[0], (T)(w[0] >> 16), (T)w[1], (T)(w[1] >> 16), (T)w[2]};
                     const T re[5] = {(T)(w[2] >> 16), (T)w[3], (T)(w[3] >> 16), (T)w[4], (T)(w[4] >> 16)};
                     const T rq[1] = {(T)w[5]};
-                    store_received_codes<Q, Q, S>((T*)a.fi, a.N_store, br, a.odd, rf);
-                    store_received_codes<Q, Q, S>((T*)a.ei, a.N_store, br, a.odd, re);
-                    store_received_codes<19, 7, S>((T*)a.fqi, a.N_store, br, a.odd, rq);
+                    store_received_codes<MEM, Q, Q, S>((T*)a.fi, a.N_store, br, a.odd, rf);
+                    store_received_codes<MEM, Q, Q, S>((T*)a.ei, a.N_store, br, a.odd, re);
+                    store_received_codes<MEM, 19, 7, S>((T*)a.fqi, a.N_store, br, a.odd, rq);
                 }
             }
         }
@@ -614,13 +687,13 @@ __global__ void __launch_bounds__(MHD ? 512 : 256)
             // the +x neighbour stores deposited for this cell by the cell one back
             // along x (if it is in the block and not solid)
             if (n64 < N) {
-                const Nbr br = neighbours(n, a.nx, a.ny, a.nz);
+                const Nbr br = neighbours<MEM>(n, a);
                 const uint32_t NX = a.nx;
                 const uint32_t src = NX <= BW ? (br.x0 == 0u ? tid + NX - 1u : tid - 1u) : (tid > 0u ? tid - 1u : XCH_NONE);
                 if (src != XCH_NONE && xfl[src]) {
-                    store_received<Q, Q, S, 0>((T*)a.fi, a.N_store, br, a.odd, xch, BW, tid);
-                    store_received<Q, Q, S, xslots<19, 19>()>((T*)a.ei, a.N_store, br, a.odd, xch, BW, tid);
-                    store_received<19, 7, S, 2 * xslots<19, 19>()>((T*)a.fqi, a.N_store, br, a.odd, xch, BW, tid);
+                    store_received<MEM, Q, Q, FS, 0>((T*)a.fi, a.N_store, br, a.odd, xch, BW, tid);
+                    store_received<MEM, Q, Q, FS, xslots<19, 19>()>((T*)a.ei, a.N_store, br, a.odd, xch, BW, tid);
+                    store_received<MEM, 19, 7, FS, 2 * xslots<19, 19>()>((T*)a.fqi, a.N_store, br, a.odd, xch, BW, tid);
                 }
             }
         }
@@ -679,7 +752,7 @@ __global__ void __launch_bounds__(256) k_update_fields(LbmArgs a) {
     const uint32_t n = (uint32_t)n64;
     const uint64_t N = a.N;
     if ((a.flags[n] & 0x1F) == 0x01) return;
-    const Nbr b = neighbours(n, a.nx, a.ny, a.nz);
+    const Nbr b = neighbours(n, a);
     R fhn[Q];
     load_ddfs<Q, Q, S>((const typename S::T*)a.fi, N, n, b, a.odd, fhn);
     R rhon, uxn, uyn, uzn;
@@ -736,7 +809,10 @@ template <class S>
 __global__ void k_codec(int dir, const void* in, void* out, uint64_t n) {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    if (dir == 0) ((uint16_t*)out)[i] = S::st(((const float*)in)[i]);
+    if (dir == 0) {  // as stream_collide does: the short form of finite values, the general one of the rest
+        const float x = ((const float*)in)[i];
+        ((uint16_t*)out)[i] = __builtin_fabsf(x) < 0x1p112f ? S::st_finite(x) : S::st(x);
+    }
     else ((float*)out)[i] = S::ld(((const uint16_t*)in)[i]);
 }
 
@@ -770,14 +846,40 @@ static hipError_t sc_ecr_impl(bool trt, bool lod, uint32_t block, const LbmArgs&
     return hipGetLastError();
 }
 
+// DDFs of up to CACHED_BYTES stay in the 256 MB last-level cache from one step
+// to the next: plain accesses and loads before the cell's flag is known; larger
+// ones stream through: nontemporal. us a step, nontemporal / plain:
+//   D3Q19 FP32   96^3  67 MB   30.6 /  21.5    D3Q15 FP16S 100^3  30 MB  20.5 /  19.3
+//               128^3 159 MB   63.5 /  45.8                160^3 123 MB  67.3 /  59.5
+//               160^3 311 MB  136.7 / 138.4                192^3 212 MB 113.3 / 114.6
+//               192^3 538 MB  212.4 / 237.6    D3Q19 FP16C 160^3 156 MB  79.3 /  60.3
+//                                                          192^3 269 MB 117.5 / 127.6
+// Streaming D3Q19 FP32 fluid: four blocks a CU, by an LDS size (more of them
+// have the memory serve more than it merges: 256^3 528 us a step with eight,
+// 517 with six, 495 with four, 510 with three). 16-bit storage, with half the
+// bytes a wavefront, is fastest with all eight (256^3 FP16C 297, 302 with six).
+constexpr uint64_t CACHED_BYTES = 192ull << 20;
+constexpr size_t FOUR_BLOCKS = 40000;
+
 template <int Q, class S>
 static hipError_t sc_impl(bool mhd, bool trt, bool lod, uint32_t block, const LbmArgs& a, hipStream_t s) {
     const uint32_t g = blocks_for(a.N, block);
     // LOD partials, and for the D3Q19 MHD variants the +x stores handed over through LDS
     // (11 values: 5 of fi, 5 of ei, 1 of fqi) plus one fluid flag per work-item
     constexpr size_t xch = Q != 19 ? 0 : (sizeof(typename S::T) == 4 ? 11 * 4 + 1 : 6 * 4 + 1);
-    const size_t sh = lod ? (size_t)block * (sizeof(typename V4<typename S::R>::T) + (mhd ? xch : 0)) : 0;
-#define ION_SC(M, T, L) hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L>), dim3(g), dim3(block), sh, s, a)
+    size_t sh = lod ? (size_t)block * (sizeof(typename V4<typename S::R>::T) + (mhd ? xch : 0)) : 0;
+    constexpr bool narrow = sizeof(typename S::R) == 4;
+    constexpr int ROWS = narrow && Q != 9 ? MEM_ROWS : MEM_CELLS, CACHED = narrow ? MEM_CACHED : MEM_CELLS;
+    const uint64_t ddfs = a.N * (Q + (mhd ? Q + 7 : 0)) * sizeof(typename S::T);
+    const bool cached = narrow && ddfs <= CACHED_BYTES;
+    if (Q == 19 && sizeof(typename S::T) == 4 && !mhd && !cached) sh = FOUR_BLOCKS;
+    const bool rows = a.nx % 64u == 0 && block % 64u == 0;
+#define ION_SC(M, T, L)                                                                                               \
+    do {                                                                                                              \
+        if (cached) hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L, false, CACHED>), dim3(g), dim3(block), sh, s, a); \
+        else if (rows) hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L, false, ROWS>), dim3(g), dim3(block), sh, s, a); \
+        else hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L>), dim3(g), dim3(block), sh, s, a);                   \
+    } while (0)
     if (mhd) {
         if (lod) { if (trt) ION_SC(true, true, true); else ION_SC(true, false, true); }
         else { if (trt) ION_SC(true, true, false); else ION_SC(true, false, false); }

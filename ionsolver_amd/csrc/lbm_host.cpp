@@ -218,6 +218,8 @@ ion::LbmArgs lbm_args(ion_handle* h) {
     a.nx = h->cfg.n_x;
     a.ny = h->cfg.n_y;
     a.nz = h->cfg.n_z;
+    a.div_x = ion::fast_div(a.nx);
+    a.div_xy = ion::fast_div(a.nx * a.ny);
     a.N = h->N;
     a.N_store = h->N;
     a.odd = (uint32_t)(h->t & 1u);
@@ -240,6 +242,10 @@ ion::LbmArgs lbm_args(ion_handle* h) {
     a.c = h->kc.c;
     a.kkge = h->kc.kkge;
     a.wq = h->kc.wq;
+    const float wm = 1.0f / (0.1875f / (1.0f / a.w - 0.5f) + 0.5f);  // TRT's second rate
+    const bool sane = std::fabs(a.w) < 1024.0f && std::fabs(a.wq) < 1024.0f && std::fabs(a.c) < 1024.0f &&
+                      (h->cfg.relaxation_time != ION_TRT || std::fabs(wm) < 1024.0f);
+    a.lim = sane ? 0x1p50f : 0.0f;
     // ils = 1.0f/lod_s(D), lod_s = (float)(bx*by*bz), sim_kernels.cl:436-440, 672
     const uint32_t nd = h->nd;
     a.ils = h->lod ? 1.0f / (float)((uint64_t)(h->cfg.n_x / nd) * (h->cfg.n_y / nd) * (h->cfg.n_z / nd)) : 0.0f;
