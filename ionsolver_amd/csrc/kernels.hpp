@@ -87,11 +87,11 @@ struct FieldArgs {
     double* judge;
     const float4* qu;       // LOD sums [n_lod]
     float* ml_ws;           // workspace of the multilevel update (MlArgs::ws_floats), or null
-    const uint32_t* mode;   // in it: whether the updates over all LOD blocks may be used [MODE_FAST, MODE_EXACT]
+    const uint32_t* mode;   // in it: whether the updates over all LOD blocks may be used [MODE_FAST, MODE_EXACT, MODE_FAST_SHIFTS]
     const float4* dense;    // in it: (q, v) at every LOD index
     uint32_t second;        // set by launch_update_e_b: another kernel runs first
 };
-enum { MODE_FAST = 0, MODE_EXACT = 1 };
+enum { MODE_FAST = 0, MODE_EXACT = 1, MODE_FAST_SHIFTS = 2 };
 // Number of blocks (judge partials) the field kernel launches for a.
 uint32_t field_blocks(const FieldArgs& a, bool fast);
 // Sums judge partials [nblocks][4] in a fixed order into out[4] (E err, E norm, B err, B norm).

@@ -110,6 +110,7 @@ __global__ void __launch_bounds__(1024) k_prep_sources(const typename V4F<R>::T*
         if (mode != nullptr) {
             mode[MODE_FAST] = base_sh >= nd * nd * nd / 32 && !any_wild;
             mode[MODE_EXACT] = base_sh >= nd * nd * nd / 4 && !any_wild;
+            mode[MODE_FAST_SHIFTS] = base_sh >= nd * nd * nd / 8 * 5 && !any_wild;
         }
     }
 }
@@ -493,13 +494,17 @@ k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
     if (a.judge != nullptr) judge_block_sums(jd, a.judge);
 }
 
-// The field update in EXACT arithmetic over all LOD blocks of depth 3 or 4.
+// The field update over all LOD blocks of depth 3 or 4, bit-identical to the
+// direct kernels: EXACT, and FAST where it has to be the direct sum (the
+// surrogate's judge and training target) or the multilevel one has no plan.
 // r / |r|^3 depends on the shift between a cell and a source only, and the
 // cells at one place of their LOD blocks see the sources of every block at the
 // same (2 nd - 1)^3 shifts: its value, rounded as in the reference, is computed
 // once for a shift and read by every pair with that shift. What is left per
 // pair are the 21 unfused multiplications and additions, in the reference's
-// order (ascending LOD index for every cell).
+// order (ascending LOD index for every cell). FAST tabulates 1 / |r|^3 and keeps
+// its 8 multiply-adds, a multiplication and shares of the differences and
+// products of a row, some 10.4 operations of 16.
 //
 // A wavefront takes the cells at (ox, oy, oz) of all blocks of a z layer of the
 // LOD grid (depth 3: of four layers), a lane four blocks in a row along x. For
@@ -516,13 +521,20 @@ k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
 // x 208 (blocks of 11 x 7 x 13 cells) 20.3 -> 6.3 ms. The direct kernels, whose
 // time goes with the number of sources, are used below a quarter of the LOD
 // blocks charged, 1024 of 4096: 128^3 with 819 sources 1.64 ms there and 2.0 here.
+// FAST 128^3 with 3511 sources 3.36 -> 1.53 ms, 256^3 16.0 -> 11.8 ms; below 5/8
+// charged the direct kernel (64^3 with 2560: 400 us both).
 //
 // Workgroups of one (oy, oz, layer) run on one XCD (block b runs on XCD b % 8),
 // ox fastest: their stores, 16 cells apart, meet in its L2.
-template <int ND>
+// The arithmetic: EXACT, and FAST as in k_update_e_b_tiled or in k_update_e_b,
+// which round (v x r).z differently.
+enum { SHIFT_EXACT = 0, SHIFT_FAST_TILED = 1, SHIFT_FAST_CELLS = 2 };
+template <int ND, int ARITH>
 __global__ void __launch_bounds__(64) k_update_e_b_shifts(FieldArgs a, uint32_t dz0, uint32_t zext, uint32_t blocks0) {
     constexpr int XG = ND / 4, PL = 64 / (XG * ND), RS = 2 * ND, ROWS = 2 * ND - 1;
-    __shared__ __align__(16) float tab[3][PL][ROWS][RS];
+    constexpr bool FAST = ARITH != SHIFT_EXACT;
+    constexpr int NC = FAST ? 1 : 3;  // 1 / |r|^3, or r / |r|^3
+    __shared__ __align__(16) float tab[NC][PL][ROWS][RS];
     const int lane = (int)threadIdx.x;
     const int bx = (int)(a.nx / ND), by = (int)(a.ny / ND), bz = (int)(a.nz / ND);
     double* const judge = a.judge == nullptr ? nullptr : a.judge + (size_t)blocks0 * 4;
@@ -561,8 +573,13 @@ __global__ void __launch_bounds__(64) k_update_e_b_shifts(FieldArgs a, uint32_t 
                     const int sx = i % RS - ND, sy = i / RS % ROWS - (ND - 1), p = i / (RS * ROWS), sz = zb * PL + p - Dz;
                     const float rx = (float)(sx * bx + ox) - 0.5f * (float)bx, ry = (float)(sy * by + oy) - 0.5f * (float)by,
                                 rz = (float)(sz * bz + oz) - 0.5f * (float)bz;
-                    const float r2 = (rx * rx + ry * ry) + rz * rz;
                     const bool own = (sx | sy | sz) == 0;
+                    if constexpr (FAST) {
+                        const float inv = __builtin_amdgcn_rsqf(__builtin_fmaf(rx, rx, __builtin_fmaf(ry, ry, rz * rz)));
+                        (&tab[0][0][0][0])[i] = own ? 0.0f : inv * inv * inv;
+                        continue;
+                    }
+                    const float r2 = (rx * rx + ry * ry) + rz * rz;
                     float fx, fy, fz;
                     if (special) {
                         const float sm = sqrt_cr(own ? 1.0f : r2);
@@ -579,33 +596,65 @@ __global__ void __launch_bounds__(64) k_update_e_b_shifts(FieldArgs a, uint32_t 
                     }
                     float* const t = &tab[0][0][0][0] + i;
                     t[0] = own ? 0.0f : fx;
-                    t[PL * ROWS * RS] = own ? 0.0f : fy;
-                    t[2 * PL * ROWS * RS] = own ? 0.0f : fz;
+                    if constexpr (!FAST) {
+                        t[PL * ROWS * RS] = own ? 0.0f : fy;
+                        t[2 * PL * ROWS * RS] = own ? 0.0f : fz;
+                    }
                 }
                 __syncthreads();
                 for (int Dy = 0; Dy < ND; Dy++) {
                     const float4* const row = (const float4*)&tab[0][zs][Y - Dy + ND - 1][4 * xg + ND];
-                    float4 A[3], B[3];  // shifts 4 xg - D .. + 3 and the four below
+                    float4 A[NC], B[NC];  // shifts 4 xg - D .. + 3 and the four below
 #pragma unroll
-                    for (int c = 0; c < 3; c++) A[c] = row[c * (PL * ROWS * RS / 4)];
+                    for (int c = 0; c < NC; c++) A[c] = row[c * (PL * ROWS * RS / 4)];
                     const cfloat_p sp = src + 4 * (Dz * ND + Dy) * ND;
+                    // cell - source; |r| is exact, so it may come from any pair of the same shift
+                    const float ry = (float)((Y - Dy) * by + oy) - 0.5f * (float)by;
+                    const float rz = (float)((Z - Dz) * bz + oz) - 0.5f * (float)bz;
+                    const float rx0 = (float)(4 * xg * bx + ox) - 0.5f * (float)bx;
+                    (void)ry, (void)rz, (void)rx0;
                     f32x16 next = *(const cf32x16_p)sp;
 #pragma unroll
                     for (int D = 0; D < ND; D += 4) {
                         const f32x16 s = next;
                         if (D + 4 < ND) next = *(const cf32x16_p)(sp + 4 * (D + 4));
 #pragma unroll
-                        for (int c = 0; c < 3; c++) B[c] = row[c * (PL * ROWS * RS / 4) - D / 4 - 1];
+                        for (int c = 0; c < NC; c++) B[c] = row[c * (PL * ROWS * RS / 4) - D / 4 - 1];
                         const uint32_t charged = (__float_as_uint(s[0]) | __float_as_uint(s[4]) | __float_as_uint(s[8]) |
                                                   __float_as_uint(s[12])) << 1;
+                        // (FAST) cell - source along x, by target - source of the groups of four
+                        float rx[7];
+                        if constexpr (FAST) {
+#pragma unroll
+                            for (int i = 0; i < 7; i++) rx[i] = __builtin_fmaf(-(float)(D + 3 - i), (float)bx, rx0);
+                        }
 #pragma unroll
                         for (int k = 0; charged != 0u && k < 4; k++) {
                             const float q = s[4 * k], vx = s[4 * k + 1], vy = s[4 * k + 2], vz = s[4 * k + 3];
+                            if constexpr (FAST) {
+                                const float cx = __builtin_fmaf(vy, rz, -(vz * ry));  // (v x r).x
+                                const float m1 = vx * rz, m2 = vx * ry;
+#pragma unroll
+                                for (int j = 0; j < 4; j++) {
+                                    const float4 w = j >= k ? A[0] : B[0];
+                                    const int e = (j - k) & 3;
+                                    const float t = q * (e == 0 ? w.x : e == 1 ? w.y : e == 2 ? w.z : w.w), x = rx[j - k + 3];
+                                    acc[j][0] = __builtin_fmaf(t, x, acc[j][0]);
+                                    acc[j][1] = __builtin_fmaf(t, ry, acc[j][1]);
+                                    acc[j][2] = __builtin_fmaf(t, rz, acc[j][2]);
+                                    acc[j][3] = __builtin_fmaf(t, cx, acc[j][3]);
+                                    acc[j][4] = __builtin_fmaf(t, __builtin_fmaf(vz, x, -m1), acc[j][4]);  // (v x r).y
+                                    const float cz = ARITH == SHIFT_FAST_TILED ? __builtin_fmaf(-vy, x, m2)  // (v x r).z
+                                                                               : __builtin_fmaf(vx, ry, -(vy * x));
+                                    acc[j][5] = __builtin_fmaf(t, cz, acc[j][5]);
+                                }
+                                continue;
+                            }
 #pragma unroll
                             for (int j = 0; j < 4; j++) {
                                 float p[3];
 #pragma unroll
-                                for (int c = 0; c < 3; c++) {
+                                for (int c = 0; c < NC; c++) {
                                     const float4 w = j >= k ? A[c] : B[c];
                                     const int e = (j - k) & 3;
                                     p[c] = e == 0 ? w.x : e == 1 ? w.y : e == 2 ? w.z : w.w;
@@ -621,7 +670,7 @@ __global__ void __launch_bounds__(64) k_update_e_b_shifts(FieldArgs a, uint32_t 
                             }
                         }
 #pragma unroll
-                        for (int c = 0; c < 3; c++) A[c] = B[c];
+                        for (int c = 0; c < NC; c++) A[c] = B[c];
                     }
                 }
             }
@@ -736,25 +785,30 @@ static FieldShape field_shape(const FieldArgs& a, bool fast) {
     return FieldShape{0, 0, 0, 0, (uint32_t)((a.N + per - 1) / per)};
 }
 
-// The shift kernel: EXACT arithmetic at LOD depth 3 and 4 without a near
-// field. Workgroups of a z layer's (oy, oz), rounded up to the 8 XCDs.
-static uint32_t shift_blocks(const FieldArgs& a) {
+// The shift kernel: LOD depth 3 and 4 without a near field; FAST arithmetic from
+// 64^3 cells on (48^3, depth 4, where too few wavefronts run: a training step
+// 1564 us source by source, 1495 here; 64^3 1720 and 1575). Workgroups of a z
+// layer's (oy, oz), rounded up to the 8 XCDs.
+static uint32_t shift_blocks(const FieldArgs& a, bool fast) {
+    if (fast && a.N < 1u << 18) return 0;
     if (a.f64 || a.near || (a.D != 3 && a.D != 4) || a.mode == nullptr || a.dense == nullptr) return 0;
+    if (a.nx >= 1u << 22 || a.ny >= 1u << 22 || a.nz >= 1u << 22) return 0;  // distances exact
     const uint32_t nd = 1u << a.D, groups = (a.ny / nd) * (a.nz / nd) * (a.D == 4 ? 16u : 2u);
     return (groups + 7) / 8 * 8 * (a.nx / nd);
 }
 
 uint32_t field_blocks(const FieldArgs& a, bool fast) {
-    return field_shape(a, fast).blocks + (fast ? 0 : shift_blocks(a));
+    return field_shape(a, fast).blocks + shift_blocks(a, fast);
 }
 
 bool over_all_blocks(const FieldArgs& a, bool fast, bool judge) {
     MlArgs m;
-    return fast ? !judge && a.judge == nullptr && a.raw == nullptr && ml_plan(a, &m) : shift_blocks(a) != 0;
+    if (fast && !judge && a.judge == nullptr && a.raw == nullptr && ml_plan(a, &m)) return true;
+    return shift_blocks(a, fast) != 0;
 }
 
 // The update over all LOD blocks first, where there is one (FAST: not for the
-// surrogate's judge and training target, which stay the plain sum), then a
+// surrogate's judge and training target, which stay the direct sum), then a
 // direct kernel; *a.mode says which of the two does the work.
 hipError_t launch_update_e_b(const FieldArgs& args, bool fast, hipStream_t s) {
     constexpr int CPT_EXACT = 1, CPT_FAST = 2;
@@ -772,15 +826,21 @@ hipError_t launch_update_e_b(const FieldArgs& args, bool fast, hipStream_t s) {
         if (e != hipSuccess) return e;
         a.second = 1;
         a.mode = args.mode + MODE_FAST;
-    }
-    if (const uint32_t nb = fast ? 0 : shift_blocks(a)) {
+    } else if (const uint32_t nb = shift_blocks(a, fast)) {
         const uint32_t nd = 1u << a.D;
         uint32_t n_lod = 0;
         for (uint32_t i = 0; i <= a.D; i++) n_lod += 1u << (3 * i);
-        a.mode = args.mode + MODE_EXACT;
+        a.mode = args.mode + (fast ? MODE_FAST_SHIFTS : MODE_EXACT);
         const uint32_t dz0 = (n_lod - nd * nd * nd) / (nd * nd), zext = (n_lod + nd * nd - 1) / (nd * nd);
-        if (a.D == 4) hipLaunchKernelGGL(k_update_e_b_shifts<16>, dim3(nb), dim3(64), 0, s, a, dz0, zext, sh.blocks);
-        else hipLaunchKernelGGL(k_update_e_b_shifts<8>, dim3(nb), dim3(64), 0, s, a, dz0, zext, sh.blocks);
+#define ION_SHIFTS(ARITH)                                                                                             \
+    do {                                                                                                              \
+        if (a.D == 4) hipLaunchKernelGGL((k_update_e_b_shifts<16, ARITH>), dim3(nb), dim3(64), 0, s, a, dz0, zext, sh.blocks); \
+        else hipLaunchKernelGGL((k_update_e_b_shifts<8, ARITH>), dim3(nb), dim3(64), 0, s, a, dz0, zext, sh.blocks);  \
+    } while (0)
+        if (!fast) ION_SHIFTS(SHIFT_EXACT);
+        else if (sh.row) ION_SHIFTS(SHIFT_FAST_TILED);
+        else ION_SHIFTS(SHIFT_FAST_CELLS);
+#undef ION_SHIFTS
         a.second = 1;
     }
     if (sh.row) {
