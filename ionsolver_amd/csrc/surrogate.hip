@@ -165,7 +165,7 @@ constexpr int BM2 = 128, BN2 = 128;
 constexpr uint32_t XCDS = 8, GM2 = 8;
 
 // Held to 128 VGPRs (the accumulators in VGPRs, not AGPRs): 4 waves per SIMD.
-template <int EPI>
+template <int EPI, bool PAIR = false>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
     k_gemm_nt_128(const __bf16* __restrict__ A, const __bf16* __restrict__ B, int M, int N, int K, int lda, int ldb,
                   GemmOut out, int m_inner) {
@@ -280,6 +280,25 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
         lagrange3((float)oz, (float)out.bz, Lz);
         hcell0 = ox + (oy + oz * out.ny) * out.nx;  // cell offset of the lane within its block
     }
+    // PAIR: the tile's 128 columns share the component, and columns 64 apart their
+    // place along x. The two waves of a row slice then take half of its rows each
+    // and all columns: a row's nine interpolations along x serve two columns,
+    // 25.5 operations a value instead of 39 (training at 128^3, no static field to
+    // read: 84 -> 73 us; inference at 256^3 waits for its loads and stores: 457 ->
+    // 450 us, with half a batch of rows in flight 473).
+    const int half = wave & 1;
+    float Lyp[2][3], Lzp[2][3];
+    uint32_t pcell[2] = {0, 0};
+    if constexpr (PAIR) {
+#pragma unroll
+        for (int w = 0; w < 2; w++) {
+            const uint32_t o = (uint32_t)(n0 + 64 * w + lane) - hc * out.cpb;
+            const uint32_t ox = o % out.bx, oy = (o / out.bx) % out.by, oz = o / (out.bx * out.by);
+            lagrange3((float)oy, (float)out.by, Lyp[w]);
+            lagrange3((float)oz, (float)out.bz, Lzp[w]);
+            pcell[w] = ox + (oy + oz * out.ny) * out.nx;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         __syncthreads();
@@ -302,10 +321,62 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
             // indices fit 32 bits (at most 2^30 cells)
             const uint32_t lnd = (uint32_t)__builtin_ctz(out.nd), mnd = out.nd - 1u;
             const uint32_t sxb = out.bx, syb = out.by * out.nx, szb = out.bz * out.nx * out.ny;
+            typedef const __attribute__((address_space(4))) float* cfar_p;  // not written by this kernel
+            if constexpr (PAIR) {
+#pragma unroll
+                for (int tb = 0; tb < 8; tb += 8) {
+                    uint32_t cell[8];
+                    uint8_t fl[8][2];
+                    float st[8][2];
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        const int m_raw = m0 + wm + i * 16 + 8 * half + tb + u;
+                        const uint32_t m = m_raw < M ? (uint32_t)m_raw : 0u;
+                        cell[u] = (uint32_t)__builtin_amdgcn_readfirstlane((m & mnd) * sxb + ((m >> lnd) & mnd) * syb +
+                                                                           (m >> (2u * lnd)) * szb);
+                        if (!train) {
+#pragma unroll
+                            for (int w = 0; w < 2; w++) {
+                                fl[u][w] = __builtin_nontemporal_load(out.flags + (cell[u] + pcell[w]));
+                                st[u][w] = raw_out ? 0.0f : __builtin_nontemporal_load(stat + (cell[u] + pcell[w]));
+                            }
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < 8; u++) {
+                        const int t = 8 * half + tb + u, m_row = m0 + wm + i * 16 + t;
+                        const cfar_p fp = (cfar_p)(out.far + ((size_t)(m_row < M ? m_row : 0) * 6 + hc) * FAR_PTS);
+                        float far[2] = {0.0f, 0.0f};
+#pragma unroll
+                        for (int zi = 0; zi < 3; zi++) {
+                            float fy[2] = {0.0f, 0.0f};
+#pragma unroll
+                            for (int yi = 0; yi < 3; yi++) {
+                                const cfar_p f = fp + zi * 9 + yi * 3;
+                                const float fx = __builtin_fmaf(Lx[2], f[2], __builtin_fmaf(Lx[1], f[1], Lx[0] * f[0]));
+#pragma unroll
+                                for (int w = 0; w < 2; w++) fy[w] = __builtin_fmaf(Lyp[w][yi], fx, fy[w]);
+                            }
+#pragma unroll
+                            for (int w = 0; w < 2; w++) far[w] = __builtin_fmaf(Lzp[w][zi], fy[w], far[w]);
+                        }
+                        if (m_row >= M) continue;
+#pragma unroll
+                        for (int w = 0; w < 2; w++) {
+                            const float v = out.alpha * Cs[(wave & 2) + w][t][lane];
+                            const uint32_t at = cell[u] + pcell[w];
+                            if (train) __builtin_nontemporal_store(v + far[w] * (out.gain / in_s), fine + at);
+                            else if ((fl[u][w] & 0x1F) != 0x01)
+                                __builtin_nontemporal_store(
+                                    raw_out ? __builtin_fmaf(rawk, v, far[w]) : (st[u][w] + in_s * sc * v) + kf * far[w], dyn + at);
+                        }
+                    }
+                }
+            }
             // rows in batches of 8: all loads of a batch (flags, static
             // field) are issued before its first store
 #pragma unroll
-            for (int tb = 0; tb < 16; tb += 8) {
+            for (int tb = 0; !PAIR && tb < 16; tb += 8) {
                 uint32_t cell[8];
                 bool valid[8];
                 uint8_t fl[8];
@@ -501,6 +572,13 @@ __global__ void k_input(const float4* __restrict__ qu, uint32_t n_top, uint32_t 
 // concatenation [a (ca channels), b (cb channels)]: row v, column
 // k = delta * (ca + cb) + ci, delta = (dx+1) + 3 (dy+1) + 9 (dz+1); columns
 // k >= 27 (ca + cb) are zero. transposed != 0 writes the [kpad][ldt] layout.
+// Eight columns (16 bytes) a work-item: channel counts are multiples of 8, so that
+// they are channels of one tensor at one delta; consecutive in v for the
+// transposed layout, whose rows are over v.
+// Bound by index arithmetic before (divisions for every value, a 2-byte access
+// each): 8.5 us a call of the forward pass at 16^3, 4.8 now; 10.2 us of a training
+// step's at 16 channels, 3.8 now.
+template <class I>
 __global__ void k_im2col(const __bf16* __restrict__ a, int ca, const __bf16* __restrict__ b, int cb, int g, int kpad,
                           __bf16* __restrict__ out, int transposed, int ldt) {
     const uint32_t cin = (uint32_t)(ca + cb), ug = (uint32_t)g, nv = ug * ug * ug, chunks = (uint32_t)kpad / 8u;
@@ -576,13 +654,6 @@ __global__ void k_up(const __bf16* __restrict__ in, int h, int c, __bf16* __rest
     const int g = 2 * h;
     const size_t total = (size_t)g * g * g * c;
     for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (size_t)gridDim.x * blockDim.x) {
-// Eight columns (16 bytes) a work-item: channel counts are multiples of 8, so that
-// they are channels of one tensor at one delta; consecutive in v for the
-// transposed layout, whose rows are over v.
-// Bound by index arithmetic before (divisions for every value, a 2-byte access
-// each): 8.5 us a call of the forward pass at 16^3, 4.8 now; 10.2 us of a training
-// step's at 16 channels, 3.8 now.
-template <class I>
         const int v = (int)(idx / c), ch = (int)(idx % c);
         const int x = (v % g) / 2, y = ((v / g) % g) / 2, z = (v / (g * g)) / 2;
         out[idx] = in[(size_t)(x + h * (y + h * z)) * c + ch];
@@ -736,6 +807,8 @@ hipError_t gemm_nt(int epi, const __bf16* A, const __bf16* B, int M, int N, int 
         const dim3 g(mi ? XCDS * GM2 * ((NT + XCDS - 1) / XCDS) * ((MT + GM2 - 1) / GM2) : MT * NT);
         if (epi == EPI_F32) hipLaunchKernelGGL(k_gemm_nt_128<EPI_F32>, g, dim3(256), 0, s, A, B, M, N, K, lda, ldb, o, mi);
         else if (epi == EPI_BF16) hipLaunchKernelGGL(k_gemm_nt_128<EPI_BF16>, g, dim3(256), 0, s, A, B, M, N, K, lda, ldb, o, mi);
+        else if ((o.cpb & 127u) == 0 && 64u % o.bx == 0)
+            hipLaunchKernelGGL((k_gemm_nt_128<EPI_HEAD, true>), g, dim3(256), 0, s, A, B, M, N, K, lda, ldb, o, mi);
         else hipLaunchKernelGGL(k_gemm_nt_128<EPI_HEAD>, g, dim3(256), 0, s, A, B, M, N, K, lda, ldb, o, mi);
         return hipGetLastError();
     }
