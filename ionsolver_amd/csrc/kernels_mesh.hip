@@ -369,7 +369,7 @@ __global__ __launch_bounds__(FLD_BLOCK) void k_static_e(Sources src, const uint8
 // A source's own cell tabulates as 0: the sums start at +0 and are never -0.
 // The kernels above are bound by the vector units' square roots and divisions;
 // this one by the table loads' latency and the scalar work of a group, beside
-// its additions (0.7 ms below). Ring and box of solid cells in 96^3, us: psi
+// its additions (0.7 ms below). A ring and a disk of solid cells in 96 x 192 x 96, us: psi
 // 24900 -> 3630, E 16000 -> 1730; the call of both, copies included, 43.1 ->
 // 8.5 ms. Bit-identical.
 // ---------------------------------------------------------------------------
