@@ -447,6 +447,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 // of the direct kernel (r / |r|^3 with the hardware reciprocal square root).
 // Sample k of an axis sits at ((k + 1/2) / 3) b - 1/2 in the block's cell
 // coordinates.
+// Sources of the neighbourhood are staged without charge and velocity: they add
+// +-0 to sums that are never -0 (no sample is a block's centre, so 1/|r| is
+// finite), and the test is made once a source instead of in each of nine rows:
+// 256^3, 4096 blocks and 3511 sources 211 -> 178 us, bound by VALU issue.
 // ---------------------------------------------------------------------------
 constexpr uint32_t FAR_TILE = 512, FAR_ROWS = 9, FAR_CHUNKS = 28, FAR_THREADS = 256;
 
@@ -473,19 +477,22 @@ __global__ void __launch_bounds__(FAR_THREADS) k_far_samples(FarArgs a) {
         const uint32_t m = min(FAR_TILE, count - base);
         __syncthreads();
         for (uint32_t i = tid; i < m; i += FAR_THREADS) {
-            s_pq[i] = a.src_pq[base + i];
-            s_vd[i] = a.src_vd[base + i];
+            float4 pq = a.src_pq[base + i], vd = a.src_vd[base + i];
+            const uint32_t d = __float_as_uint(vd.w);
+            if (d < a.nblk) {  // in-domain source: not of the 3^3 neighbourhood (own block included)
+                const int dx = (int)(d & mask) - bx, dy = (int)((d >> a.D) & mask) - by, dz = (int)(d >> (2 * a.D)) - bz;
+                if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1 && dz >= -1 && dz <= 1) {
+                    pq.w = 0.0f;
+                    vd = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                }
+            }
+            s_pq[i] = pq;
+            s_vd[i] = vd;
         }
         __syncthreads();
         if (chunk >= FAR_CHUNKS) continue;
         for (uint32_t s = chunk; s < m; s += FAR_CHUNKS) {
-            const float4 vd = s_vd[s];
-            const uint32_t d = __float_as_uint(vd.w);
-            if (d < a.nblk) {  // in-domain source: skip the 3^3 neighbourhood (own block included)
-                const int dx = (int)(d & mask) - bx, dy = (int)((d >> a.D) & mask) - by, dz = (int)(d >> (2 * a.D)) - bz;
-                if (dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1 && dz >= -1 && dz <= 1) continue;
-            }
-            const float4 pq = s_pq[s];
+            const float4 vd = s_vd[s], pq = s_pq[s];
             const float ry = py - pq.y, rz = pz - pq.z;
             const float syz = __builtin_fmaf(ry, ry, rz * rz);
             const float cx = __builtin_fmaf(vd.y, rz, -(vd.z * ry));  // (v x r).x
