@@ -854,11 +854,20 @@ static hipError_t sc_ecr_impl(bool trt, bool lod, uint32_t block, const LbmArgs&
 //               160^3 311 MB  136.7 / 138.4                192^3 212 MB 113.3 / 114.6
 //               192^3 538 MB  212.4 / 237.6    D3Q19 FP16C 160^3 156 MB  79.3 /  60.3
 //                                                          192^3 269 MB 117.5 / 127.6
+// Rows that end inside a cache line share lines between wavefronts, whose parts
+// meet in the L2 only if it keeps them: plain at every size, except large MHD FP32
+// lattices (SHARED_BYTES), of more bytes a line, and D2Q9 (us a step, nontemporal / plain):
+//   D3Q19 FP32  201 x 199 x 203 331 / 292    MHD FP16C 176 x 112 x 208 276 / 231
+//               301 x 299 x 303 1304 / 1011      FP16S 176^3           375 / 289
+//         FP16C 233 x 241 x 227 341 / 279        FP32  176 x 112 x 208 346 / 371
+//               300^3           649 / 509              144 x 112 x 144 219 / 213
+//               200^3           166 / 167    D3Q15 FP16S 232 x 240 x 224 222 / 231
+//   D2Q9  FP32  3333 x 4001     250 / 256        FP16S 3333 x 4001   162 / 177
 // Streaming D3Q19 FP32 fluid: four blocks a CU, by an LDS size (more of them
 // have the memory serve more than it merges: 256^3 528 us a step with eight,
 // 517 with six, 495 with four, 510 with three). 16-bit storage, with half the
 // bytes a wavefront, is fastest with all eight (256^3 FP16C 297, 302 with six).
-constexpr uint64_t CACHED_BYTES = 192ull << 20;
+constexpr uint64_t CACHED_BYTES = 192ull << 20, SHARED_BYTES = 512ull << 20;
 constexpr size_t FOUR_BLOCKS = 40000;
 
 template <int Q, class S>
@@ -871,14 +880,16 @@ static hipError_t sc_impl(bool mhd, bool trt, bool lod, uint32_t block, const Lb
     constexpr bool narrow = sizeof(typename S::R) == 4;
     constexpr int ROWS = narrow && Q != 9 ? MEM_ROWS : MEM_CELLS, CACHED = narrow ? MEM_CACHED : MEM_CELLS;
     const uint64_t ddfs = a.N * (Q + (mhd ? Q + 7 : 0)) * sizeof(typename S::T);
-    const bool cached = narrow && ddfs <= CACHED_BYTES;
-    if (Q == 19 && sizeof(typename S::T) == 4 && !mhd && !cached) sh = FOUR_BLOCKS;
-    const bool rows = a.nx % 64u == 0 && block % 64u == 0;
+    const bool whole = a.nx % 64u == 0 && block % 64u == 0;  // wavefronts in one row each, on whole lines
+    constexpr bool wide = sizeof(typename S::T) == 4;
+    const bool plain = narrow && (ddfs <= CACHED_BYTES || (Q != 9 && !whole && (!(mhd && wide) || ddfs <= SHARED_BYTES)));
+    if (Q == 19 && wide && !mhd && !plain) sh = FOUR_BLOCKS;
 #define ION_SC(M, T, L)                                                                                               \
     do {                                                                                                              \
-        if (cached) hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L, false, CACHED>), dim3(g), dim3(block), sh, s, a); \
-        else if (rows) hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L, false, ROWS>), dim3(g), dim3(block), sh, s, a); \
-        else hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L>), dim3(g), dim3(block), sh, s, a);                   \
+        constexpr int CELLS = ROWS == MEM_ROWS && !(M && wide) ? MEM_ROWS : MEM_CELLS; /* not reached else */        \
+        if (plain) hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L, false, CACHED>), dim3(g), dim3(block), sh, s, a); \
+        else if (whole) hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L, false, ROWS>), dim3(g), dim3(block), sh, s, a); \
+        else hipLaunchKernelGGL((k_stream_collide<Q, S, M, T, L, false, CELLS>), dim3(g), dim3(block), sh, s, a);     \
     } while (0)
     if (mhd) {
         if (lod) { if (trt) ION_SC(true, true, true); else ION_SC(true, false, true); }

@@ -22,6 +22,7 @@ pytestmark = pytest.mark.gpu
     ((2551, 4403, 1), dict(float_type=1, velocity_set=0)),
     ((128, 96, 96), dict(float_type=2, mhd=True, lod_depth=3)),
     ((104, 112, 104), dict(float_type=2, mhd=True, lod_depth=3)),
+    ((136, 144, 152), dict(float_type=2, mhd=True, lod_depth=3)),
     ((192, 112, 112), dict(float_type=1, mhd=True, lod_depth=3)),
     ((152, 136, 112), dict(float_type=0, mhd=True, lod_depth=3, charge_inlet=True)),
     ((64, 3, 1), dict(float_type=1)),
