@@ -267,7 +267,10 @@ int ion_update_e_b_noalloc(const ion_config* cfg, const ion_field_buffers* buf, 
  * is its judge: with ION_SOLVER_SURROGATE the direct kernel runs every
  * `judge_every` field steps, the relative L2 residual of the surrogate is
  * measured against it, and a residual above `tolerance` switches the next
- * `judge_every` field steps back to the direct kernel (a fallback).
+ * `judge_every` field steps back to the direct kernel (a fallback). A judged
+ * step leaves the sums that it judged by in E_dyn / B_dyn: those of
+ * ion_compute_fields to the bit in ION_FIELD_EXACT, to the rounding of the sums
+ * in ION_FIELD_FAST.
  * Needs ext_magneto_hydro, mhd_lod_depth >= 3 and an empty near-field block.
  * ------------------------------------------------------------------------ */
 typedef enum { ION_SOLVER_DIRECT = 0, ION_SOLVER_SURROGATE = 1 } ion_field_solver;
@@ -294,7 +297,10 @@ int ion_surrogate_create(ion_handle* h, const ion_surrogate_config* cfg);
  * update from the current LOD sums, Q and u. Once a surrogate exists it also
  * keeps the raw source sums (the dynamic parts before the KE / KMU scaling),
  * which are the surrogate's training and judging reference; E_dyn / B_dyn
- * are bit-identical either way. */
+ * are bit-identical either way. The raw sums are the direct kernel's in either
+ * field mode: E_stat + KE raw_E is E_dyn to the bit in ION_FIELD_EXACT, and to
+ * the rounding of the sums in ION_FIELD_FAST, which adds up E_dyn in another
+ * order where it can. */
 int ion_compute_fields(ion_handle* h);
 /* Surrogate field from the current LOD sums into E_dyn / B_dyn. */
 int ion_surrogate_infer(ion_handle* h);

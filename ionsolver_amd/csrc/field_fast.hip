@@ -98,25 +98,29 @@ struct Points {
     }
 };
 
-// Field sums of NT tiles of sample points over the sources first, first +
-// step, ... of a list, 16 at a time. |r|^2 of 16 points and 16 sources is a
-// matrix product; its lanes hold point lane & 15 and sources 4 (lane >> 4) + r,
-// which is, r by r, the left operand of the product of 1/|r|^3 with the columns
-// of the sources, and
+// Field sums of NT tiles of sample points over a list of m sources, 16 at a
+// time. |r|^2 of 16 points and 16 sources is a matrix product; its lanes hold
+// point lane & 15 and sources 4 r + (lane >> 4), which is, r by r, the left
+// operand of the product of 1/|r|^3 with the columns of four sources in a row,
+// and
 //   E = x (sum q / r^3) - sum q s / r^3,  B = (sum J / r^3) x x - sum J x s / r^3.
 // What stays on the VALU per pair are 2 instructions and a v_rsq_f32 (16 cycles
 // a wavefront, and 40 of the matrix unit, which does not run beside them) where
 // the sum of the vectors takes 21 and one (92 cycles).
+// A product adds its four terms one after the other, so a sum is taken in the
+// order of the list: a source too weak to change it leaves it as it is,
+// wherever in the list it stands.
 // The centred coordinates are below 1/2 of the distance to any source in each
 // component, so |r|^2 and the fields lose at most 2 bits to cancellation.
 template <int NT, int CAP>
-__device__ __forceinline__ void far_sums(const FarList<CAP>& list, int first, int step, int m, const Points* p, f32x4* c) {
+__device__ __forceinline__ void far_sums(const FarList<CAP>& list, int m, const Points* p, f32x4* c) {
     const int lane = (int)threadIdx.x & 63, n = min(lane & 15, 11), k = lane >> 4;
-    for (int i = first; i < m; i += step) {
-        const float sv = list.s[k][i + (lane & 15)];
+    const int row = 4 * (lane & 3) + ((lane & 15) >> 2);  // row 4 k + r: source 4 r + k
+    for (int i = 0; i < m; i += 16) {
+        const float sv = list.s[k][i + row];
         float col[4];
 #pragma unroll
-        for (int r = 0; r < 4; r++) col[r] = list.col[i + 4 * k + r][n];
+        for (int r = 0; r < 4; r++) col[r] = list.col[i + 4 * r + k][n];
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             const f32x4 r2 = __builtin_amdgcn_mfma_f32_16x16x4f32(sv, p[t].v, (f32x4){p[t].xx, p[t].xx, p[t].xx, p[t].xx}, 0, 0, 0);
@@ -212,15 +216,16 @@ __device__ void ml_tables(const MlArgs& a, uint32_t t, const float (*x)[3][ML_MA
 // Samples of the coarse levels: a workgroup takes COARSE_PTS points of a block
 // (level 2 first: its blocks have the longest source lists); the last
 // workgroups compute the tables. The sources are gathered into LDS COARSE_T
-// candidates at a time, in index order; two groups of wavefronts take every
-// second 16 and are summed at the end.
+// candidates at a time, in index order; two groups of wavefronts take those of
+// even and odd number (of the candidate, not of the source: which charges are
+// there does not move a source to the other group) and are summed at the end.
 __global__ void __launch_bounds__(COARSE_T) __attribute__((amdgpu_waves_per_eu(4))) k_ml_coarse(MlArgs a) {
     constexpr int WPG = COARSE_T / 64 / COARSE_SG;  // wavefronts of a group
     __shared__ __align__(16) union {
-        FarList<COARSE_T + 16> list;
+        FarList<COARSE_T / COARSE_SG> list[COARSE_SG];
         float tile[COARSE_T / 64][COARSE_NT][16 * 17];
     } sh;
-    __shared__ uint32_t wtot[COARSE_T / 64];
+    __shared__ uint32_t wtot[COARSE_SG][COARSE_T / 64];
     __shared__ float xs[3][3][ML_MAX_P];
     if (!multilevel(a)) return;
     uint32_t blk = blockIdx.x;
@@ -277,20 +282,22 @@ __global__ void __launch_bounds__(COARSE_T) __attribute__((amdgpu_waves_per_eu(4
             keep = !(within1(X >> shift, C[0]) && within1(Y >> shift, C[1]) && within1(Z >> shift, C[2])) &&
                    source_at(a, X, Y, Z, &s);
         }
-        const uint64_t mask = __ballot(keep);
+        static_assert(COARSE_SG == 2, "lists of even and odd candidates");
+        const uint64_t mask = __ballot(keep), even = 0x5555555555555555ull;
         __syncthreads();
-        if (lane == 0) wtot[wv] = (uint32_t)__popcll(mask);
+        if (lane < COARSE_SG) wtot[lane][wv] = (uint32_t)__popcll(mask & even << lane);
         __syncthreads();
-        int off = __popcll(mask & ((1ull << lane) - 1ull)), m = 0;
+        const int mine = lane & 1;
+        int off = __popcll(mask & even << mine & ((1ull << lane) - 1ull)), m[COARSE_SG] = {0, 0};
         for (int w = 0; w < COARSE_T / 64; w++) {
-            if (w < wv) off += (int)wtot[w];
-            m += (int)wtot[w];
+            if (w < wv) off += (int)wtot[mine][w];
+#pragma unroll
+            for (int h = 0; h < COARSE_SG; h++) m[h] += (int)wtot[h][w];
         }
-        if (keep) sh.list.put(off, s, org);
-        if (tid < 16) sh.list.pad(m, tid);
+        if (keep) sh.list[mine].put(off, s, org);
+        if (tid < 16 * COARSE_SG) sh.list[tid >> 4].pad(tid < 16 ? m[0] : m[1], tid & 15);
         __syncthreads();
-        m = __builtin_amdgcn_readfirstlane(m);
-        if (p0 < g.n) far_sums<COARSE_NT>(sh.list, 16 * grp, 16 * COARSE_SG, m, pt, acc);
+        if (p0 < g.n) far_sums<COARSE_NT>(sh.list[grp], __builtin_amdgcn_readfirstlane(grp == 0 ? m[0] : m[1]), pt, acc);
     }
     // sum of the groups, in order
     float* const out = a.ws + a.samples[li] + (size_t)blk * 6 * g.n;
@@ -421,7 +428,7 @@ __device__ __forceinline__ void far_points(const MlArgs& a, const float (*xs)[ML
             pt[t].set(x[0], x[1], x[2]);
             c[t] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
         }
-        far_sums<NT>(list, 0, 16, m, pt, c);
+        far_sums<NT>(list, m, pt, c);
 #pragma unroll
         for (int t = 0; t < NT; t++) {
             put_tile(tl, c[t]);

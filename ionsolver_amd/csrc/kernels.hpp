@@ -118,9 +118,10 @@ hipError_t launch_prep_sources(const void* qu_lod, bool f64, uint32_t lo, uint32
 // judge: with a.judge set).
 bool over_all_blocks(const FieldArgs& a, bool fast, bool judge = false);
 hipError_t launch_update_e_b(const FieldArgs& a, bool fast, hipStream_t s);
-// E_dyn = E_stat + KE raw_E, B_dyn = B_stat + KMU raw_B for fluid cells (the
-// direct kernel's own epilogue, applied to a.raw).
-hipError_t launch_combine_fields(const FieldArgs& a, hipStream_t s);
+// E_dyn and B_dyn of fluid cells beside the raw sums in a.raw, with the bits
+// that launch_update_e_b writes there without a.raw: E_stat + KE raw_E and
+// B_stat + KMU raw_B (the direct kernel's own epilogue), or the multilevel update.
+hipError_t launch_combine_fields(const FieldArgs& a, bool fast, hipStream_t s);
 hipError_t launch_sum_f64(const void* x, bool f64, const uint8_t* flags, uint64_t n, double* partial,
                           uint32_t nblocks, hipStream_t s);
 

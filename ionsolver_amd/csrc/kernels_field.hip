@@ -688,6 +688,7 @@ __global__ void __launch_bounds__(64) k_update_e_b_shifts(FieldArgs a, uint32_t 
 }
 
 __global__ void k_combine_fields(FieldArgs a) {
+    if (done_before(a)) return;
     const uint64_t n = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const uint64_t N = a.N;
     if (n >= N || (a.flags[n] & 0x1F) == 0x01) return;
@@ -786,8 +787,9 @@ static FieldShape field_shape(const FieldArgs& a, bool fast) {
 }
 
 // The shift kernel: LOD depth 3 and 4 without a near field; FAST arithmetic from
-// 64^3 cells on (48^3, depth 4, where too few wavefronts run: a training step
-// 1564 us source by source, 1495 here; 64^3 1720 and 1575). Workgroups of a z
+// 64^3 cells on (48^3, depth 4, where too few wavefronts run: a training step,
+// without the update of the fields beside its target, 1564 us source by source,
+// 1495 here; 64^3 1720 and 1575). Workgroups of a z
 // layer's (oy, oz), rounded up to the 8 XCDs.
 static uint32_t shift_blocks(const FieldArgs& a, bool fast) {
     if (fast && a.N < 1u << 18) return 0;
@@ -803,13 +805,15 @@ uint32_t field_blocks(const FieldArgs& a, bool fast) {
 
 bool over_all_blocks(const FieldArgs& a, bool fast, bool judge) {
     MlArgs m;
-    if (fast && !judge && a.judge == nullptr && a.raw == nullptr && ml_plan(a, &m)) return true;
+    if (fast && !judge && a.judge == nullptr && ml_plan(a, &m)) return true;
     return shift_blocks(a, fast) != 0;
 }
 
-// The update over all LOD blocks first, where there is one (FAST: not for the
-// surrogate's judge and training target, which stay the direct sum), then a
-// direct kernel; *a.mode says which of the two does the work.
+// The update over all LOD blocks first, where there is one (FAST: by shifts, not
+// the multilevel one, for the surrogate's judge and training target, which stay
+// the direct sum), then a direct kernel; *a.mode says which of the two does the
+// work. The target cannot be the multilevel sum: it differs by 1e-7, but the
+// network's bf16 gradients then by 1.5e-3 (128^3, 16 channels).
 hipError_t launch_update_e_b(const FieldArgs& args, bool fast, hipStream_t s) {
     constexpr int CPT_EXACT = 1, CPT_FAST = 2;
     FieldArgs a = args;
@@ -889,8 +893,19 @@ hipError_t launch_judge_reduce(const double* partial, uint32_t nblocks, double* 
     return hipGetLastError();
 }
 
-hipError_t launch_combine_fields(const FieldArgs& a, hipStream_t s) {
-    if (a.raw == nullptr) return hipErrorInvalidValue;
+hipError_t launch_combine_fields(const FieldArgs& args, bool fast, hipStream_t s) {
+    if (args.raw == nullptr) return hipErrorInvalidValue;
+    FieldArgs a = args;
+    a.second = 0;
+    a.raw = nullptr;
+    MlArgs m;
+    if (fast && ml_plan(a, &m)) {
+        const hipError_t e = launch_field_fast(m, s);
+        if (e != hipSuccess) return e;
+        a.second = 1;
+        a.mode = args.mode + MODE_FAST;
+    }
+    a.raw = args.raw;
     hipLaunchKernelGGL(k_combine_fields, dim3((uint32_t)((a.N + 255) / 256)), dim3(256), 0, s, a);
     return hipGetLastError();
 }

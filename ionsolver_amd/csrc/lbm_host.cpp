@@ -310,8 +310,9 @@ int field_update(ion_handle* h) {
     int rc = prep_sources(h, ion::over_all_blocks(f, h->field_mode == ION_FIELD_FAST));
     if (rc) return rc;
     return timed(h, 3, [&] {
-        hipError_t e = ion::launch_update_e_b(f, h->field_mode == ION_FIELD_FAST, h->stream);
-        if (e == hipSuccess && f.raw != nullptr) e = ion::launch_combine_fields(f, h->stream);
+        const bool fast = h->field_mode == ION_FIELD_FAST;
+        hipError_t e = ion::launch_update_e_b(f, fast, h->stream);
+        if (e == hipSuccess && f.raw != nullptr) e = ion::launch_combine_fields(f, fast, h->stream);
         return e;
     });
 }
@@ -324,8 +325,9 @@ ion::sur::Fields sur_fields(ion_handle* h) {
 
 // The judge's field step: the surrogate writes its raw source sums into
 // E_dyn / B_dyn, then the direct kernel compares its own sums with them while
-// it overwrites them with the direct fields (bit-identical to a direct step),
-// so no 6 x N buffer is needed for either. Residuals: relative L2 of the
+// it overwrites them with the direct fields, so no 6 x N buffer is needed for
+// either (bit-identical to a direct step in EXACT; in FAST, whose direct step
+// may be the multilevel update, equal to the rounding of the sums). Residuals: relative L2 of the
 // dynamic E and B over the fluid cells.
 int judged_field_update(ion_handle* h, double* rel_e, double* rel_b) {
     ion::FieldArgs f = field_args(h);
