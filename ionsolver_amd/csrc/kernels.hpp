@@ -94,8 +94,10 @@ struct FieldArgs {
 enum { MODE_FAST = 0, MODE_EXACT = 1, MODE_FAST_SHIFTS = 2 };
 // Number of blocks (judge partials) the field kernel launches for a.
 uint32_t field_blocks(const FieldArgs& a, bool fast);
-// Sums judge partials [nblocks][4] in a fixed order into out[4] (E err, E norm, B err, B norm).
-hipError_t launch_judge_reduce(const double* partial, uint32_t nblocks, double* out, hipStream_t s);
+// Sums judge partials [nblocks][4] in a fixed order into out[4] (E err, E norm, B err, B norm);
+// chunks: [judge_chunks(nblocks)][4] of scratch.
+uint32_t judge_chunks(uint32_t nblocks);
+hipError_t launch_judge_reduce(const double* partial, uint32_t nblocks, double* chunks, double* out, hipStream_t s);
 
 // kernels_lbm.hip
 // ecr: the SUBGRID_ECR variants (D3Q19, MHD, FP32/FP16S/FP16C)

@@ -115,6 +115,7 @@ __global__ void __launch_bounds__(1024) k_prep_sources(const typename V4F<R>::T*
     }
 }
 
+constexpr uint32_t JUDGE_CHUNK = 1024;
 constexpr uint32_t FIELD_TILE = 512;
 constexpr uint32_t FIELD_BLOCK = 256;
 
@@ -870,25 +871,39 @@ hipError_t launch_update_e_b(const FieldArgs& args, bool fast, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Judge partials [nblocks][4] -> out[4]: thread t sums the blocks t, t + 256,
-// ... of component t % 4 group, then the 64 group sums of each component are
-// added in order (a fixed order: the same residual on every run).
+// Judge partials [nblocks][4] -> out[workgroup][4], JUDGE_CHUNK partials each:
+// group t / 4 of the work-items sums the partials t / 4, t / 4 + 64, ... of the
+// chunk, then the 64 group sums of each component are added in order (a fixed
+// order: the same residual on every run).
+// Bound by the latency of its serial loads: one workgroup for all the partials of 256^3
+// took 390 us (73728 partials and 8192 zeros; they grow with the cells), chunks and
+// a second pass over their sums take 14 us.
 __global__ void __launch_bounds__(256) k_judge_reduce(const double* __restrict__ partial, uint32_t nblocks,
                                                       double* __restrict__ out) {
     __shared__ double sh[256];
     const uint32_t t = threadIdx.x, comp = t & 3u, grp = t >> 2;
+    const uint32_t first = gridDim.x == 1u ? 0u : blockIdx.x * JUDGE_CHUNK;
+    const uint32_t end = gridDim.x == 1u ? nblocks : min(nblocks, first + JUDGE_CHUNK);
     double acc = 0.0;
-    for (uint32_t b = grp; b < nblocks; b += 64u) acc += partial[(size_t)b * 4 + comp];
+    for (uint32_t b = first + grp; b < end; b += 64u) acc += partial[(size_t)b * 4 + comp];
     sh[t] = acc;
     __syncthreads();
     if (t < 4) {
         double s = 0.0;
         for (uint32_t g = 0; g < 64u; g++) s += sh[g * 4 + t];
-        out[t] = s;
+        out[(size_t)blockIdx.x * 4 + t] = s;
     }
 }
 
-hipError_t launch_judge_reduce(const double* partial, uint32_t nblocks, double* out, hipStream_t s) {
+uint32_t judge_chunks(uint32_t nblocks) { return (nblocks + JUDGE_CHUNK - 1) / JUDGE_CHUNK; }
+
+hipError_t launch_judge_reduce(const double* partial, uint32_t nblocks, double* chunks, double* out, hipStream_t s) {
+    const uint32_t n = judge_chunks(nblocks);
+    if (n > 1) {
+        hipLaunchKernelGGL(k_judge_reduce, dim3(n), dim3(256), 0, s, partial, nblocks, chunks);
+        partial = chunks;
+        nblocks = n;
+    }
     hipLaunchKernelGGL(k_judge_reduce, dim3(1), dim3(256), 0, s, partial, nblocks, out);
     return hipGetLastError();
 }

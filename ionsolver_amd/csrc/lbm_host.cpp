@@ -337,7 +337,8 @@ int judged_field_update(ion_handle* h, double* rel_e, double* rel_b) {
     if (rc) return rc;
     if (!h->judge_partials) {
         const uint32_t nb = std::max(ion::field_blocks(f, true), ion::field_blocks(f, false));
-        if ((rc = dalloc(h, (void**)&h->judge_partials, ((size_t)nb + 1) * 4 * sizeof(double)))) return rc;
+        const size_t n = (size_t)1 + nb + ion::judge_chunks(nb);
+        if ((rc = dalloc(h, (void**)&h->judge_partials, n * 4 * sizeof(double)))) return rc;
         h->judge_blocks = nb;
     }
     f.judge = h->judge_partials + 4;
@@ -346,7 +347,7 @@ int judged_field_update(ion_handle* h, double* rel_e, double* rel_b) {
         ok = h->net->infer_raw(sur_fields(h)) == 0;
         if (!ok) return hipSuccess;
         hipError_t e = ion::launch_update_e_b(f, fast, h->stream);
-        if (e == hipSuccess) e = ion::launch_judge_reduce(f.judge, ion::field_blocks(f, fast), h->judge_partials, h->stream);
+        if (e == hipSuccess) e = ion::launch_judge_reduce(f.judge, ion::field_blocks(f, fast), f.judge + (size_t)h->judge_blocks * 4, h->judge_partials, h->stream);
         return e;
     });
     if (rc) return rc;

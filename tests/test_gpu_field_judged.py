@@ -46,7 +46,7 @@ def test_raw_sums_are_the_same_by_either_route(shape, D):
         lbm.close()
 
 
-@pytest.mark.parametrize("shape,D", [((64, 64, 64), 4), ((80, 112, 48), 4), ((64, 64, 64), 3)],
+@pytest.mark.parametrize("shape,D", [((64, 64, 64), 4), ((80, 112, 48), 4), ((64, 64, 64), 3), ((128, 128, 128), 4), ((176, 112, 144), 4)],
                          ids=lambda p: "x".join(map(str, p)) if isinstance(p, tuple) else f"D{p}")
 def test_judge_of_both_routes(shape, D):
     """The gas at rest under a charge distribution: a step's LOD sums are the cells'
