@@ -110,8 +110,10 @@ struct Points {
 // A product adds its four terms one after the other, so a sum is taken in the
 // order of the list: a source too weak to change it leaves it as it is,
 // wherever in the list it stands.
-// The centred coordinates are below 1/2 of the distance to any source in each
-// component, so |r|^2 and the fields lose at most 2 bits to cancellation.
+// Of a point x and a source s that is not near, (|x|^2 + |s|^2) / |r|^2 is at
+// most 3.2 on cubic blocks and 7 on the most uneven ones that get a plan (16 x 16
+// x 5 cells), |s| / |r| at most 1.7 and 2.3: |r|^2 loses up to 1.7 and 2.8 bits to
+// cancellation, the differences of the fields about one.
 template <int NT, int CAP>
 __device__ __forceinline__ void far_sums(const FarList<CAP>& list, int m, const Points* p, f32x4* c) {
     const int lane = (int)threadIdx.x & 63, n = min(lane & 15, 11), k = lane >> 4;
@@ -688,10 +690,12 @@ __global__ void __launch_bounds__(512) k_ml_cells(MlArgs a) {
 // centre along an axis, and 1.5 sides from every cell; a function that is
 // singular at distance d straight ahead of (beside) an interval of half width
 // h is interpolated to rho^-P with rho = r + sqrt(r^2 - 1) (r + sqrt(r^2 + 1)),
-// r = d / h. The bounds below gave, against the sum at every cell in double on
-// 16^3 LOD blocks, relative errors of the far field of 2e-8 on level D, 1e-7
-// on D - 1 and 6e-8 on D - 2 (9, 9 and 10 points for cubic blocks), below the
-// 2e-7 to 4e-7 of the float sums of a direct update.
+// r = d / h. Cubic blocks get 9 points a side on level D, 10 on D - 1 and 11 on
+// D - 2; interpolated in double on 16^3 LOD blocks, the field of the sources that
+// a level takes is then off by 1e-7, 5e-8 and 2e-8 of itself (a point fewer: 4e-7,
+// 6e-7 and 1.4e-7). With the rounding of the sums the update is within 2e-7 to 4e-7
+// of the sum in double on blocks of 4 to 24 cells a side, cubic and uneven, a direct
+// one within 1.2e-6 (depth 4; 1.6e-7 to 3.4e-7 and 4.5e-7 at depth 3).
 static bool grid_of(const uint32_t b[3], uint32_t shift, uint32_t side, double tol, MlGrid* g) {
     g->shift = shift;
     g->side = side;

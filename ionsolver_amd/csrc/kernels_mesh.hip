@@ -467,7 +467,6 @@ __global__ __launch_bounds__(GRP_THREADS) void k_group(Sources src, ShiftLists o
     }
 }
 
-// NC = 1: psi of the padded lattice; NC = 3: E.
 // First and last column of fours of each batch, one batch a wavefront.
 __global__ __launch_bounds__(64) void k_batch_cols(ShiftLists l) {
     const uint32_t b = blockIdx.x, g1 = l.first[b + 1], xw = (uint32_t)l.origin[b].x;
@@ -484,6 +483,7 @@ __global__ __launch_bounds__(64) void k_batch_cols(ShiftLists l) {
     if (threadIdx.x == 0) l.cols[b] = make_int2((int)(xw + lo), (int)(xw + hi));
 }
 
+// NC = 1: psi of the padded lattice; NC = 3: E.
 template <int NC>
 __global__ __launch_bounds__(512) void k_shift_sums(Sources src, ShiftLists list, const uint8_t* flags, float* out, uint32_t nx,
                                                     uint32_t ny, uint32_t nz, float ke, uint32_t tile_q) {
