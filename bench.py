@@ -123,9 +123,6 @@ def cpu_baseline(name, seconds_hint):
                       + ", oracle built -O3 -fopenmp"}
 
 
-PSI_FLOP_PER_INTERACTION = 18  # c - p 3, |r|^2 5, sqrt 1, |r|^3 2, r.M 5, divide 1, sum 1
-
-
 def static_field_leg(scale=1.0):
     """The reference's one published timing: precompute_B of setup_deeva_test
     (src/setup.rs:395-453; 128 x 256 x 128, disk and ring magnets from
@@ -157,7 +154,6 @@ def static_field_leg(scale=1.0):
             "voxelise_s": round(t_vox, 4), "precompute_b_s": round(t_b, 4), "precompute_e_s": round(t_e, 4),
             "magnet_cells": magnets, "charged_cells": charges, "psi_interactions": inter,
             "psi_G_interactions_per_s": round(inter / t_b / 1e9, 2),
-            "psi_TFLOP_per_s": round(inter * PSI_FLOP_PER_INTERACTION / t_b / 1e12, 2),
             "reference_published_s": 37, "reference_hardware": "RTX 3060 Ti (OpenCL)",
             "speedup_vs_published": round(37.0 / t_b, 1),
             "arithmetic": "the reference's: unfused float, correctly rounded sqrt and division, same summation order"}

@@ -517,9 +517,11 @@ k_update_e_b_tiled(FieldArgs a, uint32_t TX, uint32_t TY, uint32_t TZ) {
 // block to itself, which the reference leaves out, tabulates as 0 and does the
 // same (sources that are not finite take the kernels above).
 //
-// Bound by VALU issue (4 cycles an instruction): 128^3 with 3511 sources
-// 8.2 -> 3.5 ms (21 x 4 cycles a pair are 3.0 ms), 256^3 57.2 -> 22.7 ms, 176 x 112
-// x 208 (blocks of 11 x 7 x 13 cells) 20.3 -> 6.3 ms. The direct kernels, whose
+// 128^3 with 3511 sources 8.2 -> 3.5 ms, 256^3 57.2 -> 22.7 ms, 176 x 112 x 208
+// (blocks of 11 x 7 x 13 cells) 20.3 -> 6.3 ms. Bound by VALU issue and, with few
+// wavefronts, by waits: 21.8 instructions a pair of a wavefront at 2 cycles each are
+// 73 % of the issue cycles at 256^3 and 60 % at 128^3 (8 wavefronts a SIMD in all),
+// where they would take 2.2 ms. The direct kernels, whose
 // time goes with the number of sources, are used below a quarter of the LOD
 // blocks charged, 1024 of 4096: 128^3 with 819 sources 1.64 ms there and 2.0 here.
 // FAST 128^3 with 3511 sources 3.36 -> 1.53 ms, 256^3 16.0 -> 11.8 ms; below 5/8
