@@ -40,8 +40,10 @@ FLOP_PER_INTERACTION = 35  # r 3, r^2 5, sqrt 1, cube 2, r/|r|^3 3, e 6, v x pre
 # by the factors the same counters give for ion_hbm_copy_probe's 1 GiB copy
 # (FETCH_SIZE x 2, WRITE_SIZE x 1). Kernels compiled since may differ.
 PMC_TRAFFIC = {
-    ("mhd256", "stream_collide"): 6.493e9,
-    ("mhd256-fp16c", "stream_collide"): 3.688e9,
+    ("mhd256", "stream_collide"): 6.475e9,
+    ("mhd256-fp16c", "stream_collide"): 3.668e9,
+    ("mhd256", "update_e_b_dynamic"): 0.900e9,  # FAST, in levels
+    ("mhd256-fp16c", "update_e_b_dynamic"): 0.900e9,
 }
 
 
